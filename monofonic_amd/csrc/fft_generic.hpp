@@ -1,14 +1,13 @@
-// fft_generic.hpp -- transforms of any length with a plan chosen at run time.
+// fft_generic.hpp -- transforms of lengths with a prime factor above 7.
 //
-// The tuned kernels (k_col, k_row_*, the fused LPT z stages) are compiled for
-// the transform lengths of the configured grids (fft_passes.hpp
-// MFX_COL_LENGTHS, MFX_ROW_LENGTHS).  Every other length -- any even grid
-// size the reference accepts through FFTW (src/grid_fft.cc:43-112) -- runs
-// through the kernels here: the lines of a tile live in LDS and every
-// Stockham stage reads its inputs from one LDS buffer and writes its
-// outputs to the other.  Radices 8, 4, 3 and 2 use the fixed butterflies;
-// any other prime factor p runs as a direct length-p DFT (O(p^2) per
-// butterfly), so no length needs a Bluestein pass.
+// Any even grid size the reference accepts through FFTW (src/grid_fft.cc:43-112)
+// is accepted here.  Lengths without tuned kernels (fft_passes.hpp
+// MFX_COL_LENGTHS, MFX_ROW_LENGTHS) whose prime factors are at most 7 run the
+// mixed-radix kernels (fft_mixed.hpp); the rest run through the kernels here:
+// the lines of a tile live in LDS and every Stockham stage reads its inputs
+// from one LDS buffer and writes its outputs to the other.  Radices 8, 4, 3
+// and 2 use the fixed butterflies; any other prime factor p runs as a direct
+// length-p DFT (O(p^2) per butterfly), so no length needs a Bluestein pass.
 #pragma once
 #include "fft_core.hpp"
 
@@ -123,7 +122,6 @@ __device__ cx<T>* gen_fft(cx<T>* A, cx<T>* B, const GenPlan& p, int tid, int nth
 // (thread tid works on column tid % C), both LDS buffers hold L x C values
 constexpr int GEN_THREADS = 256;
 constexpr int GEN_LDS_TILE = 65536;       // LDS per column tile aimed at
-constexpr int GEN_LDS_MAX = 160 * 1024;  // LDS of a compute unit
 
 template <typename T>
 inline int gen_col_tile(int L) {
@@ -152,36 +150,6 @@ __global__ void __launch_bounds__(GEN_THREADS)
     const cx<T> old = dst.load_old(b, colc, i);
     if (col < ncols) dst.store(b, col, i, v, old);
   }
-}
-
-// projection of a padded line (see k_col_turn): forward, keep the n modes
-// with the Nyquist mode and column zeroed, inverse
-template <typename T, class TurnA>
-__global__ void __launch_bounds__(GEN_THREADS)
-    k_col_turn_gen(TurnA a, const cx<T>* __restrict__ tw, int ncols, GenPlan plan, int C) {
-  extern __shared__ unsigned char gen_lds_raw[];
-  cx<T>* A = reinterpret_cast<cx<T>*>(gen_lds_raw);
-  cx<T>* B = A + plan.L * C;
-  const int L = plan.L;
-  const int c = threadIdx.x % C, t = threadIdx.x / C, nthr = GEN_THREADS / C;
-  const int b = blockIdx.y;
-  const int col = blockIdx.x * C + c;
-  const int colc = col < ncols ? col : ncols - 1;
-  const int nh = a.n >> 1;
-  for (int i = t; i < L; i += nthr) A[i * C + c] = a.src[(long long)b * a.sb + (long long)i * a.sp + colc];
-  __syncthreads();
-  cx<T>* r = gen_fft<false, T>(A + c, B + c, plan, t, nthr, tw, C);
-  cx<T>* other = r == A + c ? B + c : A + c;
-  const bool nyqc = colc == nh;
-  for (int i = t; i < L; i += nthr) {
-    const bool zero = ((i > nh) & (i <= a.n)) | (i == nh) | nyqc;
-    const cx<T> o = r[i * C] * a.fscale;
-    other[i * C] = zero ? mk(T(0), T(0)) : o * a.iscale;
-  }
-  __syncthreads();
-  cx<T>* q = gen_fft<true, T>(other, r, plan, t, nthr, tw, C);
-  if (col < ncols)
-    for (int i = t; i < L; i += nthr) a.out[(long long)b * a.osb + (long long)i * a.osp + col] = q[i * C];
 }
 
 // z rows: one workgroup per row of K complex (2K reals); LDS holds two

@@ -52,27 +52,6 @@ void fft_c2r_3d(Ctx& c, T* data, int n0, int n1, int n2, T scale) {
   launch_row_c2r<T>(c, n2 / 2, cd, H, (int)H, data, n2 + 2, (long long)n0 * n1, scale, "fft_z_c2r", 2 * S);
 }
 
-// The last (x) pass of the noise's forward transform writing phi(1) instead
-// of the k-space noise (ic_generator.cc:341-346,450-457): each transformed
-// value is scaled as the plain pass would store it (rounded to T) and turned
-// into phi(1) by the same per-mode function the phi(1) kernel uses, so the
-// result is bit-identical to transform-then-phi(1).  Lines along x (pos = i),
-// batch j, column kz.
-template <typename T>
-struct DstPhi1 {
-  cx<T>* phi;
-  long long sb, sp;
-  int n;
-  T scale;
-  double kfac;
-  const double* amp;
-  NoiseNorm nn;
-  __device__ __forceinline__ cx<T> load_old(int, int, int) const { return mk(T(0), T(0)); }
-  __device__ __forceinline__ void store(int b, int col, int pos, cx<T> v, cx<T>) const {
-    phi[(long long)b * sb + (long long)pos * sp + col] = phi1_value(v * scale, pos, b, col, n, kfac, amp, nn);
-  }
-};
-
 // forward transform of a real-space noise n-grid whose last pass writes
 // phi(1) into phi; the noise grid is left holding its y-stage values
 template <typename T>

@@ -4,8 +4,8 @@
 // the column kernel over tiles of adjacent columns and the z-row kernels
 // (r2c, c2r, fused c2r-product-r2c).
 #pragma once
-#include "fft_generic.hpp"
 #include "mfx_internal.hpp"
+#include "ops.hpp"
 #include "row_fft.hpp"
 
 #include <cmath>
@@ -14,6 +14,8 @@
 namespace mfx {
 
 // ------------------------------------------------------------------ config
+constexpr int CU_LDS = 160 * 1024;  // LDS of a compute unit
+
 // Tile widths of a column pass of length L (plan variant V): C, the widest
 // tile (at most 16 columns) whose exchange area fits 64 KiB of LDS, and CW =
 // 2C where C < 16 and a tile of 2C columns still fits one workgroup (1024
@@ -48,7 +50,9 @@ struct MultDev {
   __device__ __forceinline__ cx<T> eval(int i, int j, int k, int n, T kfac) const {
     T sr = 0, si = 0;
     const int idx[3] = {i, j, k};
-    for (int t = 0; t < nterms; ++t) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      if (t >= nterms) break;
       T f = 1;
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
@@ -208,6 +212,27 @@ struct DstTruncOp {
     else
       return;
     out[(long long)i * sp + (long long)b * sb + col] = value(b, col, i, v, prev);
+  }
+};
+
+// The last (x) pass of the noise's forward transform writing phi(1) instead
+// of the k-space noise (ic_generator.cc:341-346,450-457): each transformed
+// value is scaled as the plain pass would store it (rounded to T) and turned
+// into phi(1) by the same per-mode function the phi(1) kernel uses, so the
+// result is bit-identical to transform-then-phi(1).  Lines along x (pos = i),
+// batch j, column kz.
+template <typename T>
+struct DstPhi1 {
+  cx<T>* phi;
+  long long sb, sp;
+  int n;
+  T scale;
+  double kfac;
+  const double* amp;
+  NoiseNorm nn;
+  __device__ __forceinline__ cx<T> load_old(int, int, int) const { return mk(T(0), T(0)); }
+  __device__ __forceinline__ void store(int b, int col, int pos, cx<T> v, cx<T>) const {
+    phi[(long long)b * sb + (long long)pos * sp + col] = phi1_value(v * scale, pos, b, col, n, kfac, amp, nn);
   }
 };
 
@@ -535,7 +560,7 @@ unsigned pipe_grid(Ctx& c, K kernel, int block, long long nitems, size_t dyn = 0
 template <class K>
 void col_lds_prep(Ctx& c, K kernel, size_t dyn) {
   if (dyn <= 65536) return;
-  MFX_REQUIRE(dyn <= (size_t)GEN_LDS_MAX, "column tile too large for one compute unit's LDS");
+  MFX_REQUIRE(dyn <= (size_t)CU_LDS, "column tile too large for one compute unit's LDS");
   int& done = c.lds_attr[(const void*)kernel];
   if (done < (int)dyn) {
     MFX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn));
@@ -669,30 +694,23 @@ inline bool col_plan_alt(int L) {
 }
 
 // ------------------------------------------------------------------ lengths without tuned kernels
-// A kernel whose dynamic LDS exceeds the default 64 KiB is allowed more once.
-template <class K>
-void gen_lds_prep(Ctx& c, K kernel, size_t lds) {
-  MFX_REQUIRE(lds <= (size_t)GEN_LDS_MAX, "transform length too long for one compute unit's LDS");
-  if (lds <= 65536) return;
-  int& done = c.lds_attr[(const void*)kernel];
-  if (done < (int)lds) {
-    MFX_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    done = (int)lds;
-  }
-}
-
+// (mixed_kernels.hip: run-time schedules)
 template <typename T, bool INV, class Src, class Dst>
-void launch_col_gen(Ctx& c, int L, Src s, Dst d, int ncols, int nbatch, const char* name, double bytes) {
-  const GenPlan plan = gen_plan(L);
-  const int C = gen_col_tile<T>(L);
-  const size_t lds = 2 * (size_t)L * C * sizeof(cx<T>);
-  auto k = k_col_gen<T, INV, Src, Dst>;
-  gen_lds_prep(c, k, lds);
-  LaunchScope ls(c, name, bytes);
-  hipLaunchKernelGGL(k, dim3((ncols + C - 1) / C, nbatch), dim3(GEN_THREADS), lds, c.stream, s, d, c.twiddles<T>(L),
-                     ncols, plan, C);
-  check_launch(name);
-}
+void launch_col_any(Ctx& c, int L, Src s, Dst d, int ncols, int nbatch, const char* name, double bytes);
+template <typename T>
+void launch_turn_any(Ctx& c, int L, const TurnArgs<T>& a, int ncols, int nbatch, const char* name, double bytes);
+template <typename T>
+void launch_row_r2c_any(Ctx& c, int K, const T* src, long long spitch, cx<T>* dst, long long dpitch, int hout,
+                        long long nrows, T scale, const char* name, double bytes);
+template <typename T>
+void launch_row_c2r_any(Ctx& c, int K, const cx<T>* src, long long spitch, int hin, T* dst, long long dpitch,
+                        long long nrows, T scale, const char* name, double bytes);
+template <typename T>
+void launch_row_c2r_part_any(Ctx& c, int K, const cx<T>* src, long long spitch, int hin, double* out, long long nrows,
+                             T scale, int idim, double lunit, int kind, double qoff, const char* name, double bytes);
+template <typename T>
+void launch_row_prod_any(Ctx& c, int K, const cx<T>* a, const cx<T>* b, long long spitch, int hin, cx<T>* dst,
+                         long long dpitch, int hout, long long nrows, const char* name, double bytes);
 
 template <typename T, bool INV, class Src, class Dst>
 void launch_col(Ctx& c, int L, Src s, Dst d, int ncols, int nbatch, const char* name, double bytes) {
@@ -704,7 +722,7 @@ void launch_col(Ctx& c, int L, Src s, Dst d, int ncols, int nbatch, const char* 
     MFX_COL_LENGTHS(MFX_CASE)
 #undef MFX_CASE
     default:
-      launch_col_gen<T, INV>(c, L, s, d, ncols, nbatch, name, bytes);
+      launch_col_any<T, INV>(c, L, s, d, ncols, nbatch, name, bytes);
   }
 }
 
@@ -724,7 +742,7 @@ void launch_col_pad(Ctx& c, int L, Src s, Dst d, int ncols, int nbatch, const ch
     MFX_PAD_LENGTHS(MFX_CASE)
 #undef MFX_CASE
     default:
-      launch_col_gen<T, INV>(c, L, s, d, ncols, nbatch, name, bytes);
+      launch_col_any<T, INV>(c, L, s, d, ncols, nbatch, name, bytes);
   }
 }
 
@@ -798,17 +816,8 @@ void launch_turn(Ctx& c, int L, const TurnArgs<T>& a, int ncols, int nbatch, con
     return;
     MFX_PAD_LENGTHS(MFX_CASE)
 #undef MFX_CASE
-    default: {
-      const GenPlan plan = gen_plan(L);
-      const int C = gen_col_tile<T>(L);
-      const size_t lds = 2 * (size_t)L * C * sizeof(cx<T>);
-      auto k = k_col_turn_gen<T, TurnArgs<T>>;
-      gen_lds_prep(c, k, lds);
-      LaunchScope ls(c, name, bytes);
-      hipLaunchKernelGGL(k, dim3((ncols + C - 1) / C, nbatch), dim3(GEN_THREADS), lds, c.stream, a,
-                         c.twiddles<T>(L), ncols, plan, C);
-      check_launch(name);
-    }
+    default:
+      launch_turn_any<T>(c, L, a, ncols, nbatch, name, bytes);
   }
 }
 
@@ -866,7 +875,7 @@ void launch_multi(Ctx& c, int L, const M& a, long long sp, int ncols, int nbatch
 #undef MFX_CASE
     default:
       for (int o = 0; o < a.no; ++o)
-        launch_col_gen<T, INV>(c, L, MultiSrc<T, M>{a, o}, MultiDst<T, M>{a, o}, ncols, nbatch, name, bytes / a.no);
+        launch_col_any<T, INV>(c, L, MultiSrc<T, M>{a, o}, MultiDst<T, M>{a, o}, ncols, nbatch, name, bytes / a.no);
   }
 }
 
@@ -1073,27 +1082,13 @@ void launch_row_prod_K(Ctx& c, const cx<T>* a, const cx<T>* b, long long spitch,
   check_launch(name);
 }
 
-// rows of a length without tuned kernels go to the generic kernel (GEN)
+// rows of a length without tuned kernels go to the run-time schedules (GEN)
 #define MFX_ROW_SWITCH(K, CALL, GEN) \
   switch (K) {                       \
     MFX_ROW_LENGTHS(CALL)            \
     default:                         \
       GEN;                           \
   }
-
-// one generic row kernel launch: one workgroup per row
-#define MFX_GEN_ROW_LAUNCH(KERNEL, NBUF, ...)                                                       \
-  do {                                                                                              \
-    const GenPlan plan_ = gen_plan(K);                                                              \
-    const size_t lds_ = gen_row_lds<T>(K, NBUF);                                                    \
-    auto k_ = KERNEL<T>;                                                                            \
-    gen_lds_prep(c, k_, lds_);                                                                      \
-    MFX_REQUIRE(nrows < (1LL << 31), "too many rows for one launch");                               \
-    LaunchScope ls_(c, name, bytes);                                                                \
-    hipLaunchKernelGGL(k_, dim3((unsigned)nrows), dim3(GEN_THREADS), lds_, c.stream, __VA_ARGS__, plan_, \
-                       c.twiddles<T>(K), c.twiddles<T>(2 * K));                                     \
-    check_launch(name);                                                                             \
-  } while (0)
 
 template <typename T>
 void launch_row_r2c(Ctx& c, int K, const T* src, long long spitch, cx<T>* dst, long long dpitch, int hout,
@@ -1102,7 +1097,7 @@ void launch_row_r2c(Ctx& c, int K, const T* src, long long spitch, cx<T>* dst, l
   case KK:                                                                                        \
     launch_row_r2c_K<T, KK>(c, src, spitch, dst, dpitch, hout, nrows, scale, name, bytes);       \
     return;
-  MFX_ROW_SWITCH(K, MFX_CASE, MFX_GEN_ROW_LAUNCH(k_row_r2c_gen, 2, src, spitch, dst, dpitch, hout, scale))
+  MFX_ROW_SWITCH(K, MFX_CASE, launch_row_r2c_any<T>(c, K, src, spitch, dst, dpitch, hout, nrows, scale, name, bytes))
 #undef MFX_CASE
 }
 
@@ -1113,7 +1108,7 @@ void launch_row_c2r(Ctx& c, int K, const cx<T>* src, long long spitch, int hin, 
   case KK:                                                                                        \
     launch_row_c2r_K<T, KK>(c, src, spitch, hin, dst, dpitch, nrows, scale, name, bytes);        \
     return;
-  MFX_ROW_SWITCH(K, MFX_CASE, MFX_GEN_ROW_LAUNCH(k_row_c2r_gen, 2, src, spitch, hin, dst, dpitch, scale))
+  MFX_ROW_SWITCH(K, MFX_CASE, launch_row_c2r_any<T>(c, K, src, spitch, hin, dst, dpitch, nrows, scale, name, bytes))
 #undef MFX_CASE
 }
 
@@ -1135,7 +1130,7 @@ void launch_row_c2r_part(Ctx& c, int K, const cx<T>* src, long long spitch, int 
     launch_row_c2r_part_K<T, KK>(c, src, spitch, hin, out, nrows, scale, idim, lunit, kind, qoff, name, bytes); \
     return;
   MFX_ROW_SWITCH(K, MFX_CASE,
-                 MFX_GEN_ROW_LAUNCH(k_row_c2r_part_gen, 2, src, spitch, hin, out, scale, idim, lunit, kind, qoff))
+                 launch_row_c2r_part_any<T>(c, K, src, spitch, hin, out, nrows, scale, idim, lunit, kind, qoff, name, bytes))
 #undef MFX_CASE
 }
 
@@ -1146,7 +1141,7 @@ void launch_row_prod(Ctx& c, int K, const cx<T>* a, const cx<T>* b, long long sp
   case KK:                                                                                          \
     launch_row_prod_K<T, KK>(c, a, b, spitch, hin, dst, dpitch, hout, nrows, name, bytes);        \
     return;
-  MFX_ROW_SWITCH(K, MFX_CASE, MFX_GEN_ROW_LAUNCH(k_row_prod_gen, 4, a, b, spitch, hin, dst, dpitch, hout))
+  MFX_ROW_SWITCH(K, MFX_CASE, launch_row_prod_any<T>(c, K, a, b, spitch, hin, dst, dpitch, hout, nrows, name, bytes))
 #undef MFX_CASE
 }
 

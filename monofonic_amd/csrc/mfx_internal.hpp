@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "fft_core.hpp"
+#include "mix_plan.hpp"
 
 namespace mfx {
 
@@ -87,6 +88,8 @@ struct Ctx {
   int num_cus();
   std::map<const void*, int> occupancy;  // resident workgroups per CU, per kernel
   std::map<const void*, int> lds_attr;   // dynamic LDS bytes allowed, per kernel
+  // schedules of lengths without tuned kernels, per (length, element size, use)
+  std::map<std::tuple<int, int, int>, MixCfg> mix;
   ~Ctx();
   template <typename T>
   const cx<T>* twiddles(int L);
