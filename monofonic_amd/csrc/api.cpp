@@ -128,6 +128,7 @@ struct mfx_conv {
   size_t lpt_bytes = 0;
   int lpt_path = MFX_LPT_AUTO;  // requested 3LPT path
   int lpt_chosen = MFX_LPT_AUTO;  // path the 3LPT workspace was reserved for
+  int lpt_refused = 0;  // lowest LPT order whose engine workspace did not fit (0: none)
   mfx_grid* fbuf = nullptr;  // convolve3 intermediate (convolution.hh:469)
 };
 
@@ -902,14 +903,43 @@ static void lpt_reserve(mfx_conv* cv, int order) {
   }
 }
 
-static void lpt_fused(mfx_conv* cv, mfx_grid* phi, mfx_grid* phi2, mfx_grid* phi3, mfx_grid* A3[3], int order) {
+// Whether the fused engine runs this convolver's sources at LPT order `order`,
+// its workspace reserved: always at grid sizes with tuned z stages; at the
+// other sizes it supports (the mixed-radix stages: 2LPT and stored 3LPT) where
+// the workspace takes at most a third of the free device memory, so that
+// programs that hold many generators keep room for them (any room with 8 GiB to
+// spare where the caller asked for the stored path).  Otherwise the convolve
+// sequence, whose workspace is a fraction of it.  A refusal is remembered until
+// the path is set again: the decision does not change between calls.
+static bool lpt_engine_ready(mfx_conv* cv, int order) {
+  Ctx& c = cv->ctx->c;
   if (!lpt_fused_supported(cv->n)) {
-    // a grid size the engine is not compiled for: the same fields from the
-    // convolve sequence
+    if (cv->lpt_refused && order >= cv->lpt_refused) return false;
+    if (!lpt_mixed_supported(c, cv->n, cv->prec)) return false;
+    if (order > 2 && cv->lpt_path == MFX_LPT_STREAMED) return false;
+    const size_t need = lpt_workspace_bytes(cv->n, cv->prec, order, true);
+    if (cv->lpt_bytes < need) {
+      size_t fr = 0, tot = 0;
+      MFX_HIP(hipMemGetInfo(&fr, &tot));
+      fr += cv->lpt_bytes;
+      const bool fits = cv->lpt_path == MFX_LPT_STORED ? need + ((size_t)8 << 30) <= fr : need <= fr / 3;
+      if (!fits) {
+        cv->lpt_refused = order;
+        return false;
+      }
+    }
+    if (order > 2) cv->lpt_chosen = MFX_LPT_STORED;
+  }
+  lpt_reserve(cv, order);
+  return true;
+}
+
+static void lpt_fused(mfx_conv* cv, mfx_grid* phi, mfx_grid* phi2, mfx_grid* phi3, mfx_grid* A3[3], int order) {
+  if (!lpt_engine_ready(cv, order)) {
+    // the same fields from the convolve sequence
     lpt_sequence(cv, phi, phi2, phi3, A3, order);
     return;
   }
-  lpt_reserve(cv, order);
   grid_forward(phi, true);
   phi2->space = MFX_KSPACE;
   if (order > 2) {
@@ -933,6 +963,7 @@ int mfx_conv_set_lpt_path(mfx_conv* cv, int path) {
     MFX_REQUIRE(path == MFX_LPT_AUTO || path == MFX_LPT_STREAMED || path == MFX_LPT_STORED, "invalid LPT path");
     cv->lpt_path = path;
     cv->lpt_chosen = MFX_LPT_AUTO;
+    cv->lpt_refused = 0;
   });
 }
 
@@ -1604,8 +1635,7 @@ extern "C" int mfx_icgen_create(mfx_ctx* c, const mfx_icgen_params* p, mfx_icgen
       // FP32 this keeps the realisation within one GPU's HBM); they stay valid
       // until the next run.
       const size_t ncell = p->n * p->n * p->n, npart = ncell * (size_t)ic->overload;
-      if (ic->conv && p->use_fused_lpt && !p->own_particles && lpt_fused_supported((int)p->n)) {
-        lpt_reserve(ic->conv, p->lpt_order);
+      if (ic->conv && p->use_fused_lpt && !p->own_particles && lpt_engine_ready(ic->conv, p->lpt_order)) {
         if (ic->conv->lpt_bytes >= 6 * npart * sizeof(double)) {
           ic->part_in_ws = true;
           for (int w = 0; w < 6; ++w) ic->part[w] = (double*)ic->conv->lpt_ws + w * npart;

@@ -28,41 +28,13 @@
 // the 3a intermediates).  The intermediates are truncated to the n-grid and
 // padded back by one projection pass per axis on their y/z slot (turn).
 #include "fft_passes.hpp"
-#include "ops.hpp"
+#include "lpt_common.hpp"
 
 #include <type_traits>
 
 namespace mfx {
 
 // ------------------------------------------------------------------ z stage
-// Y arrays of one field: 0 -> Y0, 1 -> Yx, 2 -> Yy, 3 -> Yxx, 4 -> Yxy, 5 -> Yyy
-template <typename T>
-struct FieldY {
-  const cx<T>* y[6];
-};
-
-// Hessian component (a,b) -> Y array and kz power
-constexpr int hess_idx(int a, int b) {
-  return (a > b) ? hess_idx(b, a)
-                 : (a == 0 && b == 0) ? 3
-                 : (a == 1 && b == 1) ? 5
-                 : (a == 2 && b == 2) ? 0
-                 : (a == 0 && b == 1) ? 4
-                 : (a == 0 && b == 2) ? 1
-                                      : 2;
-}
-constexpr int hess_pz(int a, int b) { return (a == 2) + (b == 2); }
-
-template <typename T>
-struct KzMul {
-  int n, pz;
-  T kfac, sgn;
-  __device__ __forceinline__ T operator()(int k) const {
-    T g = kval<T>(k, n, kfac, 1);
-    return pz == 0 ? sgn : (pz == 1 ? sgn * g : sgn * g * g);
-  }
-};
-
 // compile-time loop: f(std::integral_constant<int, O>) for O = B .. N-1
 template <int B, int N, class F>
 __device__ __forceinline__ void static_for(F&& f) {
@@ -333,12 +305,6 @@ __global__ void __launch_bounds__(RowLanes<K>::THREADS)
 // outputs overwrite the intermediates' rows -- phi3 -> I1, A3x -> I2,
 // A3y -> I3, A3z -> I4 -- all of which are consumed before the first output
 // is written.
-namespace cs {
-// stored component order xx, yy, zz, xy, xz, yz
-constexpr int ca[6] = {0, 1, 2, 0, 0, 1};
-constexpr int cb[6] = {0, 1, 2, 1, 2, 2};
-}  // namespace cs
-
 template <typename T, int K>
 __global__ void __launch_bounds__(RowLanes<K>::THREADS)
     k_lpt_zC(FieldY<T> f2, const cx<T>* R, long long rstride, cx<T>* I1, cx<T>* I2, cx<T>* I3, cx<T>* I4,
@@ -483,15 +449,19 @@ void launch_zC2_K(Ctx& c, const FieldY<T>& f1, const FieldY<T>& f2, int i, cx<T>
   check_launch("lpt_zC2");
 }
 
-#define MFX_LPT_KSWITCH(K, CALL)                                          \
-  switch (K) {                                                            \
-    MFX_PAD_K_LENGTHS(CALL)                                               \
-    default:                                                              \
-      throw Error(1, "unsupported padded length " + std::to_string(2 * (K))); \
+// padded lengths outside the list: the mixed-radix stage (MIX), or none
+#define MFX_LPT_KSWITCH(K, CALL, MIX) \
+  switch (K) {                        \
+    MFX_PAD_K_LENGTHS(CALL)           \
+    default:                          \
+      MIX;                            \
   }
+#define MFX_LPT_NONE(K) throw Error(1, "unsupported padded length " + std::to_string(2 * (K)))
 
-// the fused engine is compiled for the padded row lengths K = 3n/4 of
-// MFX_PAD_K_LENGTHS; other grid sizes take the convolve sequence
+// the fused engine has tuned z stages for the padded row lengths K = 3n/4 of
+// MFX_PAD_K_LENGTHS; other grid sizes run the mixed-radix ones (2LPT and the
+// stored 3LPT path) where the padded length has a schedule, else the convolve
+// sequence
 bool lpt_fused_supported(int n) {
   if (n % 4 != 0) return false;
   switch (3 * n / 4) {
@@ -503,6 +473,13 @@ bool lpt_fused_supported(int n) {
     default:
       return false;
   }
+}
+
+bool lpt_mixed_supported(Ctx& c, int n, int prec) {
+  if (n % 4 != 0) return false;
+  const int m = 3 * n / 2;
+  return prec == 4 ? mix_cfg<float>(c, m, MIX_COL).ok && mix_cfg<float>(c, m, MIX_Z).ok
+                   : mix_cfg<double>(c, m, MIX_COL).ok && mix_cfg<double>(c, m, MIX_Z).ok;
 }
 
 // ------------------------------------------------------------------ host orchestration
@@ -664,7 +641,9 @@ void lpt_sources(Ctx& c, const cx<T>* phi, cx<T>* phi2, cx<T>* phi3, cx<T>* a3x,
   case KK:                                                                                                    \
     launch_zA_K<T, KK>(c, fphi, E.T2[6], Iz, three, E.R, (long long)l.treal, l.hp, l.h, n, E.kfac, nrows, bytes); \
     break;
-    MFX_LPT_KSWITCH(K, MFX_CASE)
+    MFX_LPT_KSWITCH(K, MFX_CASE,
+                    launch_zA_mix<T>(c, fphi, E.T2[6], Iz, three, E.R, (long long)l.treal, l.hp, l.h, n, E.kfac, nrows,
+                                     bytes))
 #undef MFX_CASE
   }
   if (!three) {
@@ -689,7 +668,8 @@ void lpt_sources(Ctx& c, const cx<T>* phi, cx<T>* phi2, cx<T>* phi3, cx<T>* a3x,
   case KK:                                                                                             \
     launch_zC_K<T, KK>(c, E.fy(0), E.R, (long long)l.treal, Ir, l.hp, l.h, n, E.kfac, nrows, bytes); \
     break;
-    MFX_LPT_KSWITCH(K, MFX_CASE)
+    MFX_LPT_KSWITCH(K, MFX_CASE,
+                    launch_zC_mix<T>(c, E.fy(0), E.R, (long long)l.treal, Ir, l.hp, l.h, n, E.kfac, nrows, bytes))
 #undef MFX_CASE
     cx<T>* out[4] = {phi3, a3x, a3y, a3z};
     for (int q = 0; q < 4; ++q) E.forward(Ir[q], out[q], true);
@@ -712,7 +692,7 @@ void lpt_sources(Ctx& c, const cx<T>* phi, cx<T>* phi2, cx<T>* phi3, cx<T>* a3x,
   case KK:                                                                                            \
     launch_zC1_K<T, KK>(c, fphi, fphi2, Ir, Ir[0], l.hp, l.h, n, E.kfac, nrows, bytes); \
     break;
-    MFX_LPT_KSWITCH(K, MFX_CASE)
+    MFX_LPT_KSWITCH(K, MFX_CASE, MFX_LPT_NONE(K))
 #undef MFX_CASE
   }
   E.forward(Ir[0], phi3, true);
@@ -724,7 +704,7 @@ void lpt_sources(Ctx& c, const cx<T>* phi, cx<T>* phi2, cx<T>* phi3, cx<T>* a3x,
   case KK:                                                                                        \
     launch_zC2_K<T, KK>(c, fphi, fphi2, i, Ir[1 + i], l.hp, l.h, n, E.kfac, nrows, bytes); \
     break;
-    MFX_LPT_KSWITCH(K, MFX_CASE)
+    MFX_LPT_KSWITCH(K, MFX_CASE, MFX_LPT_NONE(K))
 #undef MFX_CASE
     E.forward(Ir[1 + i], A3[i], true);
   }

@@ -1,13 +1,16 @@
 """The mixed-radix kernels (fft_mixed.hpp) at the lengths and row counts where
 their schedules change: two to four stages, each radix, an odd number of rows
 (a pair with one row), tiles with fewer columns than their width, the longest
-lines."""
+lines; and the fused LPT engine on the padded lengths that run them."""
 import numpy as np
 import pytest
 
 from conftest import rel_max, rel_rms
+from helpers import random_kspace_field
 
 pytestmark = pytest.mark.gpu
+
+BOX = 100.0
 
 
 # a transform of length L errs by about eps log2(L) in the rms: 1e-13 is 40
@@ -33,3 +36,49 @@ def test_transforms_vs_numpy(ctx, shape, prec, tol):
     back = g.download()
     assert rel_max(back[:, :, :n2], x) < 20 * tol
     assert np.all(back[:, :, n2:] == 0)
+
+
+def _fields(M, ctx, orc, n, prec):
+    phi_h = random_kspace_field(orc, n, n, slope=-3.0)
+    phi = M.Grid_FFT(ctx, n, BOX, prec, initialspace=M.kspace_id)
+    phi.upload(phi_h)
+    out = [M.Grid_FFT(ctx, n, BOX, prec, initialspace=M.kspace_id) for _ in range(5)]
+    return phi_h, phi, out
+
+
+# padded lengths 30, 42, 54, 60, 90, 150, 180: schedules of one to three stages
+# before the fixed last radix (6 in FP32, 3 in FP64)
+@pytest.mark.parametrize("n", [20, 28, 36, 40, 60, 100, 120])
+@pytest.mark.parametrize("prec,rms,mx", [("double", 1e-12, 1e-10), ("float", 2e-5, 2e-3)])
+@pytest.mark.parametrize("order", [2, 3])
+def test_lpt_engine_vs_oracle(ctx, orc, n, prec, rms, mx, order):
+    import monofonic_amd as M
+    print(f"mixed lpt engine n={n} {prec} order={order}", flush=True)
+    phi_h, phi, (phi2, phi3, *A3) = _fields(M, ctx, orc, n, prec)
+    conv = M.OrszagConvolver(ctx, n, BOX, prec)
+    if order == 2:
+        conv.lpt_sources(phi, phi2, order=2)
+    else:
+        conv.lpt_sources(phi, phi2, phi3, tuple(A3), order=3)
+        assert conv.lpt_path == "stored"  # the engine ran, not the convolve sequence
+    r2, r3, rA = orc.lpt_terms(phi_h, BOX, order)
+    pairs = [(phi2, r2)] + ([(phi3, r3)] + list(zip(A3, rA)) if order == 3 else [])
+    for got, ref in pairs:
+        assert rel_rms(got.kdata(), orc.kview(ref)) < rms
+        assert rel_max(got.kdata(), orc.kview(ref)) < mx
+
+
+@pytest.mark.parametrize("n", [20, 28, 60, 100])
+def test_lpt_streamed_request_keeps_the_sequence(ctx, orc, n):
+    """the mixed-radix stages have no streamed 3LPT path: asked for it, such a
+    size runs the convolve sequence, which the engine agrees with"""
+    import monofonic_amd as M
+    phi_h, phi, (phi2, phi3, *A3) = _fields(M, ctx, orc, n, "double")
+    conv = M.OrszagConvolver(ctx, n, BOX, "double")
+    conv.set_lpt_path("streamed")
+    conv.lpt_sources(phi, phi2, phi3, tuple(A3), order=3)
+    seq = [g.kdata().copy() for g in (phi2, phi3, *A3)]
+    conv.set_lpt_path("stored")
+    conv.lpt_sources(phi, phi2, phi3, tuple(A3), order=3)
+    for g, s in zip((phi2, phi3, *A3), seq):
+        assert rel_rms(g.kdata(), s) < 1e-12
