@@ -6,7 +6,8 @@
 // time by a parallel twist in LDS; every pair of consecutive uniforms is one
 // attempt of Leva's ratio method (gsl_ran_ugaussian_ratio_method), evaluated
 // for all 312 pairs of a block at once, and the accepted deviates are ranked
-// by wave ballots so that they land in the cube in stream order.
+// by wave ballots so that they land in the cube in stream order.  Where there are
+// few cubes the stream and its evaluation run side by side (k_music1_few).
 // The global mean is taken with a double-double sum, i.e. the correctly
 // rounded exact sum, and subtracted in double (ctor at :35-66).
 //
@@ -244,6 +245,159 @@ __global__ void __launch_bounds__(256) k_music1_cubes(T* data, int n, int nc, in
   if (tid == 0) part[icube] = red[0];
 }
 
+// The next 624 words of the stream from the last 624, by one wave.  Words 227
+// apart depend on one another, so there are three rounds; the wave's own LDS
+// accesses run in order, and the fence keeps the compiler from moving a round's
+// reads above the writes before it.
+__device__ __forceinline__ void mt_next(const unsigned* old, unsigned* nxt, int lane) {
+  constexpr int W = MT_N - MT_M;  // 227
+  auto round = [&](int k0, int k1, const unsigned* far) {
+    // all reads of a round before its writes: the compiler cannot tell the
+    // blocks apart and would wait for each write's reads in turn
+    unsigned y[4], f[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int kc = k0 + lane + 64 * r, k = kc < k1 ? kc : k1 - 1;
+      y[r] = (old[k] & 0x80000000u) | ((k + 1 < MT_N ? old[k + 1] : nxt[0]) & 0x7fffffffu);
+      f[r] = far[k];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int k = k0 + lane + 64 * r;
+      if (k < k1) nxt[k] = f[r] ^ (y[r] >> 1) ^ mt_mag(y[r]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+  };
+  round(0, W, old + MT_M);
+  round(W, 2 * W, nxt - W);
+  round(2 * W, MT_N, nxt - W);
+}
+
+// The fill for few cubes.  A cube's stream is serial, so with no more cubes than
+// a couple for each compute unit its latency decides: one wave produces a group
+// of MU_G blocks while MU_E others evaluate the group before it, MU_CHUNKS / MU_E
+// chunks of 64 pairs each, with one barrier for each group where k_music1_cubes
+// has six for each block.  FP32 grids in the IC driver's form: 64^3 (8 cubes) 222
+// -> 98 us, 256^3 (512 cubes) 279 -> 204 us; 512^3 (4096 cubes) 1.08 -> 1.44 ms,
+// where the FP64 arithmetic of the evaluation decides and k_music1_cubes keeps
+// every wave on it.
+constexpr int MU_G = 4, MU_PAIRS = MU_G * MT_N / 2, MU_CHUNKS = 20, MU_E = 10;
+static_assert(64 * MU_CHUNKS >= MU_PAIRS && MU_CHUNKS % MU_E == 0, "the chunks cover a group, evenly shared");
+
+template <typename T, bool SUMS>
+__global__ void __launch_bounds__(64 * (1 + MU_E)) k_music1_few(T* data, int n, int nc, int cs, int lcs,
+                                                                 int wrap, const long* seedp, dd* part) {
+  constexpr int C = MU_CHUNKS / MU_E;
+  __shared__ unsigned words[2][MU_G][MT_N];             // two groups of blocks
+  __shared__ __align__(16) unsigned wcnt[2][MU_CHUNKS];  // accepted pairs per chunk, for alternating groups
+  const long baseseed = *seedp;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const long long icube = blockIdx.x;
+  const int ci = (int)(icube / ((long long)nc * nc)), cj = (int)((icube / nc) % nc), ck = (int)(icube % nc);
+  // the seeded state is the block before the first: the last of group 1
+  if (tid == 0) mt_seed(words[1][MU_G - 1], (unsigned long)(baseseed + icube));
+  __syncthreads();
+  auto produce = [&](int g) {
+    const unsigned* old = words[g ^ 1][MU_G - 1];
+#pragma unroll 1
+    for (int q = 0; q < MU_G; ++q) {
+      mt_next(old, words[g][q], lane);
+      old = words[g][q];
+    }
+  };
+  if (wave == 0) produce(0);
+  __syncthreads();
+  // a cube holds cs^3 < 2^31 values (checked on the host), so the stream
+  // positions are 32-bit; they split into cell indices by shifts when
+  // cs = 2^lcs and by division otherwise (lcs < 0)
+  const unsigned ucs = (unsigned)cs, cnt = ucs * ucs * ucs;
+  const int pitch = n + 2;
+  T* const cube = data + (((long long)ci * cs) * n + (long long)cj * cs) * pitch + (long long)ck * cs;
+  unsigned count = 0;
+  dd acc{0.0, 0.0};
+  for (int g = 0; count < cnt; g ^= 1) {
+    double val[C];
+    unsigned long long ok[C];
+    if (wave == 0) {
+      produce(g ^ 1);
+    } else {
+      // chunk q of the group: pairs 64 q + lane, in stream order across the
+      // group (a block's words are consecutive)
+      const unsigned* w = words[g][0];
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const int chunk = (wave - 1) * C + c, p = 64 * chunk + lane;
+        bool acc_p = false;
+        val[c] = 0;
+        if (p < MU_PAIRS) {
+          const double U1 = mt_temper(w[2 * p]) / 4294967296.0;
+          const double U2 = mt_temper(w[2 * p + 1]) / 4294967296.0;
+          acc_p = leva(U1, U2, &val[c]);
+        }
+        ok[c] = __ballot(acc_p);
+        if (lane == 0) wcnt[g][chunk] = (unsigned)__popcll(ok[c]);
+      }
+    }
+    __syncthreads();  // the counts of this group, the words of the next
+    unsigned before = count, total = 0;
+#pragma unroll
+    for (int q = 0; q < MU_CHUNKS; ++q) {
+      const unsigned m = wcnt[g][q];
+      before += q < (wave - 1) * C ? m : 0u;
+      total += m;
+    }
+    if (wave > 0) {
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const unsigned e = before + (unsigned)__popcll(ok[c] & ((1ull << lane) - 1ull));
+        before += (unsigned)__popcll(ok[c]);
+        if (!((ok[c] >> lane) & 1ull)) continue;
+        if (e < cnt) {
+          unsigned kk, jj, ii;
+          if (lcs >= 0) {
+            kk = e & (ucs - 1u);
+            jj = (e >> lcs) & (ucs - 1u);
+            ii = e >> (2 * lcs);
+          } else {
+            const unsigned q = e / ucs;
+            kk = e - q * ucs;
+            jj = q % ucs;
+            ii = q / ucs;
+          }
+          // a row index below 2^24 and one 64-bit multiply-add
+          const unsigned row = __umul24(ii, (unsigned)n) + jj;
+          T sv = T(val[c]);
+          cube[(unsigned long long)row * (unsigned)pitch + kk] = sv;
+          if constexpr (SUMS) {
+            if (wrap) {
+              // m * sv exactly as the pair (p, e) of a two-product
+              const double m = (double)(music1_mult(n, nc, cs, ci, (int)ii) * music1_mult(n, nc, cs, cj, (int)jj) *
+                                        music1_mult(n, nc, cs, ck, (int)kk));
+              const double pr = m * (double)sv;
+              acc = dd_add(dd_add(acc, pr), fma(m, (double)sv, -pr));
+            } else {
+              acc = dd_add(acc, (double)sv);
+            }
+          }
+        }
+      }
+    }
+    count += total;
+  }
+  if constexpr (!SUMS) return;
+  // the threads' sums, then those of the waves
+  __shared__ dd red[1 + MU_E];
+#pragma unroll
+  for (int s = 32; s > 0; s >>= 1) acc = dd_add2(acc, dd{__shfl_down(acc.hi, s), __shfl_down(acc.lo, s)});
+  if (lane == 0) red[wave] = acc;
+  __syncthreads();
+  if (tid == 0) {
+    for (int w = 1; w <= MU_E; ++w) acc = dd_add2(acc, red[w]);
+    part[icube] = acc;
+  }
+}
+
 __global__ void k_dd_mean(const dd* part, long long nparts, double inv_count, double* mean) {
   __shared__ dd red[256];
   dd acc{0.0, 0.0};
@@ -364,12 +518,13 @@ void music1_fill(Ctx& c, T* data, int n, const long* dseed, int cubesize, int ze
   } restore{c, prof};
   {
     LaunchScope ls(c, "music1_cubes", (double)n * n * n * sizeof(T));
-    if (zeromean == 2)
-      hipLaunchKernelGGL((k_music1_cubes<T, false>), dim3((unsigned)ncube), dim3(256), 0, c.stream, data, n, nc, cs,
-                         lcs, wrap, dseed, part);
-    else
-      hipLaunchKernelGGL((k_music1_cubes<T, true>), dim3((unsigned)ncube), dim3(256), 0, c.stream, data, n, nc, cs,
-                         lcs, wrap, dseed, part);
+    // two cubes for each compute unit: the line between latency and arithmetic
+    // (k_music1_few: 512 cubes 204 against 279 us, 4096 cubes 1.44 against 1.08 ms)
+    const bool few = ncube <= 2LL * c.num_cus();
+    auto k = few ? (zeromean == 2 ? k_music1_few<T, false> : k_music1_few<T, true>)
+                 : (zeromean == 2 ? k_music1_cubes<T, false> : k_music1_cubes<T, true>);
+    hipLaunchKernelGGL(k, dim3((unsigned)ncube), dim3(few ? 64 * (1 + MU_E) : 256), 0, c.stream, data, n, nc, cs, lcs,
+                       wrap, dseed, part);
     check_launch("music1_cubes");
   }
   const long long tot = (long long)n * n * (n + 2);

@@ -73,3 +73,16 @@ def test_threefry_fill(ctx, orc):
     got = g.rdata()
     ref = orc.threefry_fill(n, 3)[:, :, :n]
     assert np.max(np.abs(got - ref)) < 1e-14 * np.max(np.abs(ref))
+
+
+# 512 cubes is the last count the few-cubes fill takes on a 256-unit device; cubes
+# of 2^3 and 3^3 values need a fraction of one block, 40^3 many groups of blocks
+@pytest.mark.parametrize("n,cs", [(128, 16), (128, 14), (64, 6), (8, 2), (16, 3), (64, 40), (4, 1)])
+@pytest.mark.parametrize("prec", ["double", "float"])
+def test_music1_fill_either_side_of_the_cube_count(ctx, orc, n, cs, prec):
+    import monofonic_amd as M
+    print(f"music1 n={n} cs={cs} {prec}", flush=True)
+    g = M.Grid_FFT(ctx, n, 100.0, prec)
+    M.RNG_music(4711, cs).Fill_Grid(g)
+    # bit for bit, the subtracted mean and its roundings included
+    assert np.array_equal(g.rdata(), orc.music1_fill(n, 4711, cs, f32=prec == "float")[:, :, :n])
