@@ -86,3 +86,18 @@ def test_music1_fill_either_side_of_the_cube_count(ctx, orc, n, cs, prec):
     M.RNG_music(4711, cs).Fill_Grid(g)
     # bit for bit, the subtracted mean and its roundings included
     assert np.array_equal(g.rdata(), orc.music1_fill(n, 4711, cs, f32=prec == "float")[:, :, :n])
+
+
+# seeds at the edges of the 32-bit word that seeds the table's stream, and odd
+# and even numbers of draws after the last increment
+@pytest.mark.parametrize("seed", [0, 1, 2147483647, 2147483653, 4294967296, -7])
+@pytest.mark.parametrize("n", [4, 22])
+def test_ngenic_fill_seed_edges(ctx, orc, seed, n):
+    import monofonic_amd as M
+    g = M.Grid_FFT(ctx, n, 100.0, "double")
+    M.RNG_ngenic(seed).Fill_Grid(g)
+    got = g.kdata()
+    ref = orc.kview(orc.ngenic_fill(n, orc.ngenic_seedtable(n, seed)))
+    # the streams are exact; log, sin and cos may differ in the last place
+    assert np.max(np.abs(got - ref)) < 1e-14 * np.max(np.abs(ref))
+    assert np.array_equal(got == 0, ref == 0)
