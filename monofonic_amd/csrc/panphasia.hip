@@ -584,6 +584,28 @@ PanSizes pan_sizes(const PanDesc& d, int n) {
   return s;
 }
 
+// Unnormalised r2c (FFTW's) of the 84 coefficient fields, np^3 each, one after
+// another in memory: their rows are contiguous, so are their x-planes, and an
+// x-plane of a field is np (np/2 + 1) adjacent columns of x lines.  One launch a
+// pass over as many fields as a grid's y dimension holds (84 x np / 32768 launches
+// a pass; one field at a time took 252 launches of 8 us where the data of a 128^3
+// cube takes 3 to 4 us each).
+template <typename T>
+static void pan_r2c(Ctx& c, T* coef, int np) {
+  const long long H = np / 2 + 1, plane = np * H, field = plane * np;
+  cx<T>* k = reinterpret_cast<cx<T>*>(coef);
+  const int step = std::max(1, std::min(84, 32768 / np));
+  for (int l = 0; l < 84; l += step) {
+    const int m = std::min(step, 84 - l);
+    cx<T>* f = k + l * field;
+    const double S = (double)m * field * sizeof(cx<T>);
+    launch_row_r2c<T>(c, np / 2, reinterpret_cast<T*>(f), np + 2, f, H, (int)H, (long long)m * np * np, T(1),
+                      "fft_z_r2c", 2 * S);
+    col_pass_plain<T, false>(c, np, f, f, plane, H, (int)H, m * np, T(1), "fft_y_fwd", 2 * S);
+    col_pass_plain<T, false>(c, np, f, f, field, plane, (int)plane, m, T(1), "fft_x_fwd", 2 * S);
+  }
+}
+
 template <typename T>
 void panphasia_noise(Ctx& c, const PanDesc& d, int n, cx<T>* wn) {
   MFX_REQUIRE(n % 2 == 0 && n > 0, "Panphasia: even grid size required");
@@ -639,53 +661,54 @@ void panphasia_noise(Ctx& c, const PanDesc& d, int n, cx<T>* wn) {
     owned.push_back(p);
     return p;
   };
-  auto up = [&](const void* h, size_t bytes) {
-    void* p = dalloc(bytes);
-    MFX_HIP(hipMemcpyAsync(p, h, bytes, hipMemcpyHostToDevice, c.stream));
-    return p;
+  // All tables and per-level lists travel in one copy: their bytes are laid out
+  // in one host buffer, whose device copy holds each at the same offset.
+  std::vector<char> host;
+  auto lay = [&](const void* h, size_t bytes) {
+    const size_t at = (host.size() + 15) / 16 * 16;
+    host.resize(at + bytes);
+    if (bytes) std::memcpy(host.data() + at, h, bytes);
+    return at;
   };
+  const size_t orp = lay(rp.data(), sizeof(int) * rp.size()), oci = lay(ci.data(), sizeof(int) * ci.size()),
+               ocv = lay(cv.data(), sizeof(double) * cv.size()), ocp = lay(cp.data(), sizeof(int) * cp.size()),
+               orr = lay(rr.data(), sizeof(int) * rr.size()), orv = lay(rv.data(), sizeof(double) * rv.size()),
+               otabi = lay(tabi.data(), sizeof(int) * tabi.size()),
+               oprank = lay(prank.data(), sizeof(int) * prank.size()),
+               osph = lay(sph.data(), sizeof(cx<double>) * sph.size());
+  std::vector<size_t> ocoord[3], ochild[3];
+  size_t operm[3];
+  for (int q = 0; q < 3; ++q) {
+    for (int L = 0; L <= lmax; ++L) {
+      ocoord[q].push_back(lay(ax[q].coord[L].data(), sizeof(unsigned long long) * ax[q].coord[L].size()));
+      if (L < lmax) ochild[q].push_back(lay(ax[q].child[L].data(), sizeof(int) * ax[q].child[L].size()));
+    }
+    operm[q] = lay(ax[q].perm.data(), sizeof(int) * ax[q].perm.size());
+  }
   try {
-    const int* drp = (const int*)up(rp.data(), sizeof(int) * rp.size());
-    const int* dci = (const int*)up(ci.data(), sizeof(int) * ci.size());
-    const double* dcv = (const double*)up(cv.data(), sizeof(double) * cv.size());
-    const int* dcp = (const int*)up(cp.data(), sizeof(int) * cp.size());
-    const int* drr = (const int*)up(rr.data(), sizeof(int) * rr.size());
-    const double* drv = (const double*)up(rv.data(), sizeof(double) * rv.size());
-    int* dtabi = (int*)up(tabi.data(), sizeof(int) * tabi.size());
-    int* dprank = (int*)up(prank.data(), sizeof(int) * prank.size());
-    cx<double>* dsph = (cx<double>*)up(sph.data(), sizeof(cx<double>) * sph.size());
+    char* const dev = (char*)dalloc(host.size());
+    MFX_HIP(hipMemcpyAsync(dev, host.data(), host.size(), hipMemcpyHostToDevice, c.stream));
+    const int* dprank = (const int*)(dev + oprank);
+    const cx<double>* dsph = (const cx<double>*)(dev + osph);
     double* root = (double*)dalloc(sizeof(double) * 84);
     double* lev[2] = {(double*)dalloc(sizeof(double) * 84 * maxcells), (double*)dalloc(sizeof(double) * 84 * maxcells)};
     // coefficient fields and their transforms in the grid's precision (the
     // reference computes Panphasia in real_t: float in single-precision builds)
     T* coef = (T*)dalloc(sizeof(T) * 84 * (size_t)fstride);
-    // per-level lists
-    std::vector<const unsigned long long*> dcoord[3];
-    std::vector<const int*> dchild[3];
-    const int* dperm[3];
-    for (int q = 0; q < 3; ++q) {
-      for (int L = 0; L <= lmax; ++L) {
-        dcoord[q].push_back((const unsigned long long*)up(ax[q].coord[L].data(),
-                                                          sizeof(unsigned long long) * ax[q].coord[L].size()));
-        dchild[q].push_back(L < lmax ? (const int*)up(ax[q].child[L].data(), sizeof(int) * ax[q].child[L].size())
-                                     : nullptr);
-      }
-      dperm[q] = (const int*)up(ax[q].perm.data(), sizeof(int) * ax[q].perm.size());
-    }
     LaunchScope ls(c, "panphasia_cells", 0);
     PanLevelArgs a{};
-    a.rp = drp;
-    a.ci = dci;
-    a.cv = dcv;
-    a.cp = dcp;
-    a.rr = drr;
-    a.rv = drv;
-    a.tabi = dtabi;
+    a.rp = (const int*)(dev + orp);
+    a.ci = (const int*)(dev + oci);
+    a.cv = (const double*)(dev + ocv);
+    a.cp = (const int*)(dev + ocp);
+    a.rr = (const int*)(dev + orr);
+    a.rv = (const double*)(dev + orv);
+    a.tabi = (const int*)(dev + otabi);
     a.np = np;
     a.fstride = fstride;
     a.coef = coef;
     a.coef_f32 = sizeof(T) == 4;
-    for (int q = 0; q < 3; ++q) a.perm[q] = dperm[q];
+    for (int q = 0; q < 3; ++q) a.perm[q] = (const int*)(dev + operm[q]);
     // root cell
     a.mode = 2;
     a.cnt[0] = a.cnt[1] = a.cnt[2] = 1;
@@ -702,8 +725,8 @@ void panphasia_noise(Ctx& c, const PanDesc& d, int n, cx<T>* wn) {
       a.parent = parent;
       a.level = (unsigned long long)L;
       for (int q = 0; q < 3; ++q) {
-        a.coord[q] = dcoord[q][L];
-        a.child[q] = dchild[q][L];
+        a.coord[q] = (const unsigned long long*)(dev + ocoord[q][L]);
+        a.child[q] = (const int*)(dev + ochild[q][L]);
         a.cnt[q] = (int)ax[q].coord[L].size();
         a.cnt1[q] = (int)ax[q].coord[L + 1].size();
       }
@@ -716,8 +739,7 @@ void panphasia_noise(Ctx& c, const PanDesc& d, int n, cx<T>* wn) {
       check_launch("panphasia_cells");
       parent = lev[L & 1];
     }
-    // r2c of the 84 coefficient fields (FFTW's unnormalised transform)
-    for (int l = 0; l < 84; ++l) fft_r2c_3d<T>(c, coef + (size_t)l * fstride, np, np, np, T(1));
+    pan_r2c<T>(c, coef, np);
     const long long nm = (long long)n * n * (n / 2 + 1);
     fill<T>(c, (T*)wn, 2 * nm, T(0));
     {
