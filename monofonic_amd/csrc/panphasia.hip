@@ -376,7 +376,7 @@ constexpr int kPanCellsPerGroup = 3;
 
 __global__ void __launch_bounds__(256) k_pan_cells(PanLevelArgs a) {
   constexpr int CPG = kPanCellsPerGroup;
-  __shared__ double g[CPG][672];
+  __shared__ double g[CPG][693];  // 672 used: the slots start 42 banks apart
   __shared__ double diff[CPG][84];
   __shared__ long long dst[CPG][8];  // per child: output offset, -1 if not needed
   const int t = threadIdx.x;
@@ -462,6 +462,34 @@ __global__ void __launch_bounds__(256) k_pan_cells(PanLevelArgs a) {
   // parity blocks -> children: child c, coefficient l = sqrt(1/8) sum_j
   // (-1)^popcount(c & (j ^ parity(l))) block_j[l]
   const double nrm = sqrt(0.125);
+  if (a.mode == 1) {
+    // Into the coefficient fields: a thread forms the eight children of one
+    // (cell, l) from one read of its blocks, and the cells of a workgroup, which
+    // are neighbours along z, are adjacent lanes, so that a store covers runs of
+    // up to six values of a field rather than single ones (64 fields at once).
+    // The cell solve of a 512^3 FP32 grid takes 20 ms, 32 ms with one value of 64
+    // fields in each store.
+    for (int q = t; q < 84 * CPG; q += 256) {
+      const int s2 = q % CPG, l = q / CPG, pb = pbits[l];
+      double v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = g[s2][84 * j + l];
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const long long o = dst[s2][c];
+        if (o < 0) continue;
+        double e = 0.0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) e += (__popc((unsigned)(c & (j ^ pb))) & 1) ? -v[j] : v[j];
+        const double val = nrm * e;
+        if (a.coef_f32)
+          ((float*)a.coef)[(long long)l * a.fstride + o] = (float)val;
+        else
+          ((double*)a.coef)[(long long)l * a.fstride + o] = val;
+      }
+    }
+    return;
+  }
   for (int q = t; q < (root ? 84 : 672 * CPG); q += 256) {
     const int s2 = q / 672, ql = q % 672;
     const int c = ql / 84, l = ql % 84, pb = pbits[l];
@@ -472,14 +500,7 @@ __global__ void __launch_bounds__(256) k_pan_cells(PanLevelArgs a) {
       const double v = g[s2][84 * j + l];
       e += (__popc((unsigned)(c & (j ^ pb))) & 1) ? -v : v;
     }
-    const double val = nrm * e;
-    if (a.mode == 1) {
-      if (a.coef_f32)
-        ((float*)a.coef)[(long long)l * a.fstride + o] = (float)val;
-      else
-        ((double*)a.coef)[(long long)l * a.fstride + o] = val;
-    } else
-      a.out[o + l] = val;
+    a.out[o + l] = nrm * e;
   }
 }
 
