@@ -562,8 +562,7 @@ __global__ void __launch_bounds__(256)
       const double wr = wxr * bz.x - wxi * bz.y, wi = wxr * bz.y + wxi * bz.x;
       ar[u] = ar[u] + (wr * f.x - wi * f.y);
       ai[u] = ai[u] + (wr * f.y + wi * f.x);
-      const double aw = hypot(wr, wi);
-      W[u] = W[u] + aw * aw;
+      W[u] = W[u] + (wr * wr + wi * wi);
     }
   }
   const double pi = 4.0 * atan(1.0);
