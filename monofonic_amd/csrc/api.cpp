@@ -1901,6 +1901,20 @@ static void icgen_device_run(mfx_icgen* ic) {
     }
     tmp->space = MFX_RSPACE;
   };
+  // the six components of the sc load, as many together as fit the 256 MiB
+  // memory-side cache with room to spare: a pass over a group then finds the
+  // previous pass's values there, and small grids take three launches instead of
+  // eighteen of about 5 us each (64^3); grids beyond the cache go one by one
+  auto components = [&](auto* comp, long long ws) {
+    using TT = decltype(comp->x);
+    const int fit = (int)((160ll << 20) / (ws * (long long)sizeof(*comp)));
+    const int g = fit >= 6 ? 6 : fit >= 3 ? 3 : fit >= 2 ? 2 : 1;
+    int codes[6];
+    for (int w = 0; w < 6; ++w) codes[w] = (w % 3) | okind(w) << 2;
+    for (int w = 0; w < 6; w += g)
+      fft_c2r_particle_set<TT>(ic->ctx->c, (TT*)(comp + w * ws), (int)p.n, (TT)norm_fac(tmp), g, ic->part + w,
+                               codes + w, 1.0);
+  };
   // bcc/fcc/rsc (particle_generator.hh:499-543,597-638): sublattice l of
   // component w holds its field at the cell positions shifted by
   // kLatticeShift[l] (shift_field by the difference to the previous
@@ -1939,12 +1953,10 @@ static void icgen_device_run(mfx_icgen* ic) {
                            (const cx<float>*)P(phi2), (const cx<float>*)P(phi3), (const cx<float>*)P(A3[0]),
                            (const cx<float>*)P(A3[1]), (const cx<float>*)P(A3[2]), (int)p.n, p.boxlen, p.lpt_order,
                            ic->vfact, 1.0, plt_tab, plt_ng, gr);
-        for (int w = 0; w < 6; ++w)
-          if (ic->overload == 1 && sp == 0 && !p.baryons)
-            fft_c2r_particles<float>(ic->ctx->c, (float*)((cx<float>*)ic->comp6 + w * ws), (int)p.n,
-                                     (float)norm_fac(tmp), ic->part[w], w % 3, 1.0, okind(w));
-          else
-            sublattices(w, (cx<float>*)ic->comp6 + w * ws, sp);
+        if (ic->overload == 1 && !p.baryons)
+          components((cx<float>*)ic->comp6, ws);
+        else
+          for (int w = 0; w < 6; ++w) sublattices(w, (cx<float>*)ic->comp6 + w * ws, sp);
       }
     } else {
       assemble6<double>(ic->ctx->c, (cx<double>*)ic->comp6, ws, (const cx<double>*)phi->d,
@@ -1957,12 +1969,10 @@ static void icgen_device_run(mfx_icgen* ic) {
                             (const cx<double>*)P(phi2), (const cx<double>*)P(phi3), (const cx<double>*)P(A3[0]),
                             (const cx<double>*)P(A3[1]), (const cx<double>*)P(A3[2]), (int)p.n, p.boxlen,
                             p.lpt_order, ic->vfact, 1.0, plt_tab, plt_ng, gr);
-        for (int w = 0; w < 6; ++w)
-          if (ic->overload == 1 && sp == 0 && !p.baryons)
-            fft_c2r_particles<double>(ic->ctx->c, (double*)((cx<double>*)ic->comp6 + w * ws), (int)p.n,
-                                      norm_fac(tmp), ic->part[w], w % 3, 1.0, okind(w));
-          else
-            sublattices(w, (cx<double>*)ic->comp6 + w * ws, sp);
+        if (ic->overload == 1 && !p.baryons)
+          components((cx<double>*)ic->comp6, ws);
+        else
+          for (int w = 0; w < 6; ++w) sublattices(w, (cx<double>*)ic->comp6 + w * ws, sp);
       }
     }
     density();

@@ -9,7 +9,7 @@
 // and 2 use the fixed butterflies; any other prime factor p runs as a direct
 // length-p DFT (O(p^2) per butterfly), so no length needs a Bluestein pass.
 #pragma once
-#include "fft_core.hpp"
+#include "fft_passes.hpp"
 
 namespace mfx {
 
@@ -249,16 +249,16 @@ __global__ void __launch_bounds__(GEN_THREADS)
 // c2r writing FP64 particles (see k_row_c2r_part)
 template <typename T>
 __global__ void __launch_bounds__(GEN_THREADS)
-    k_row_c2r_part_gen(const cx<T>* src, long long spitch, int hin, double* out, T scale, int idim, double lunit,
-                       int kind, double qoff, GenPlan plan, const cx<T>* __restrict__ twK,
-                       const cx<T>* __restrict__ twM) {
+    k_row_c2r_part_gen(const cx<T>* src, long long spitch, int hin, PartOut po, T scale, double lunit, double qoff,
+                       GenPlan plan, const cx<T>* __restrict__ twK, const cx<T>* __restrict__ twM) {
   MFX_GEN_ROW_PROLOGUE(T)
   const int n = 2 * K;
   gen_load_half(gr.A, src + row * spitch, hin, K);
   const cx<T>* z = gr.c2r();
-  const int i = (int)(row / n), j = (int)(row % n);
+  const int rw = (int)(row / n), w = rw / n, i = rw - w * n, j = (int)(row - (long long)rw * n);
+  const int code = po.code(w), idim = code & 3, kind = code >> 2;
   const double qrow = (double)(idim == 0 ? i : j) / (double)n * lunit + qoff;
-  double* o = out + row * n;
+  double* o = po.array(w) + ((long long)i * n + j) * n;
   for (int m = tid; m < K; m += GEN_THREADS) {
     double f0 = (double)(z[m].x * scale), f1 = (double)(z[m].y * scale);
     if (kind == 0) {

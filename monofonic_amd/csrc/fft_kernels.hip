@@ -26,6 +26,19 @@
 namespace mfx {
 
 // ------------------------------------------------------------------ 3D transforms
+// The x pass of `narr` grids, one after another, of L planes of `plane` values: the
+// (j, kz) of a plane are adjacent, so they form one range of columns.  Tiles then
+// start at whole multiples of their width, on 128-byte lines where the plane
+// stride is one, and no row ends in a partial tile (at 512^3 a row of 257 columns
+// took 17 tiles of 16, each across two lines; X_FIGURES).
+template <typename T, bool INV>
+static void launch_x(Ctx& c, int L, const cx<T>* src, cx<T>* dst, long long plane, T scale, int narr,
+                     const char* name, double bytes) {
+  MFX_REQUIRE(plane < (1LL << 31), "plane too large for one pass");
+  launch_col<T, INV>(c, L, SrcPlain<T>{src, plane * L, plane}, DstPlain<T>{dst, plane * L, plane, scale}, (int)plane,
+                     narr, name, bytes);
+}
+
 template <typename T>
 void fft_r2c_3d(Ctx& c, T* data, int n0, int n1, int n2, T scale) {
   MFX_REQUIRE(n2 % 2 == 0, "r2c requires an even last dimension");
@@ -35,8 +48,7 @@ void fft_r2c_3d(Ctx& c, T* data, int n0, int n1, int n2, T scale) {
   launch_row_r2c<T>(c, n2 / 2, data, n2 + 2, cd, H, (int)H, (long long)n0 * n1, T(1), "fft_z_r2c", 2 * S);
   launch_col<T, false>(c, n1, SrcPlain<T>{cd, (long long)n1 * H, H}, DstPlain<T>{cd, (long long)n1 * H, H, T(1)},
                        (int)H, n0, "fft_y_fwd", 2 * S);
-  launch_col<T, false>(c, n0, SrcPlain<T>{cd, H, (long long)n1 * H}, DstPlain<T>{cd, H, (long long)n1 * H, scale},
-                       (int)H, n1, "fft_x_fwd", 2 * S);
+  launch_x<T, false>(c, n0, cd, cd, (long long)n1 * H, scale, 1, "fft_x_fwd", 2 * S);
 }
 
 template <typename T>
@@ -45,8 +57,7 @@ void fft_c2r_3d(Ctx& c, T* data, int n0, int n1, int n2, T scale) {
   const long long H = n2 / 2 + 1;
   cx<T>* cd = reinterpret_cast<cx<T>*>(data);
   const double S = (double)n0 * n1 * (n2 + 2) * sizeof(T);
-  launch_col<T, true>(c, n0, SrcPlain<T>{cd, H, (long long)n1 * H}, DstPlain<T>{cd, H, (long long)n1 * H, T(1)},
-                      (int)H, n1, "fft_x_inv", 2 * S);
+  launch_x<T, true>(c, n0, cd, cd, (long long)n1 * H, T(1), 1, "fft_x_inv", 2 * S);
   launch_col<T, true>(c, n1, SrcPlain<T>{cd, (long long)n1 * H, H}, DstPlain<T>{cd, (long long)n1 * H, H, T(1)},
                       (int)H, n0, "fft_y_inv", 2 * S);
   launch_row_c2r<T>(c, n2 / 2, cd, H, (int)H, data, n2 + 2, (long long)n0 * n1, scale, "fft_z_c2r", 2 * S);
@@ -63,8 +74,8 @@ void fft_r2c_phi1(Ctx& c, T* wn, int n, T scale, cx<T>* phi, double boxlen, cons
   launch_row_r2c<T>(c, n / 2, wn, n + 2, cd, H, (int)H, (long long)n * n, T(1), "fft_z_r2c", 2 * S);
   launch_col<T, false>(c, n, SrcPlain<T>{cd, (long long)n * H, H}, DstPlain<T>{cd, (long long)n * H, H, T(1)},
                        (int)H, n, "fft_y_fwd", 2 * S);
-  DstPhi1<T> d{phi, H, (long long)n * H, n, scale, 2.0 * M_PI / boxlen, amp, nn};
-  launch_col<T, false>(c, n, SrcPlain<T>{cd, H, (long long)n * H}, d, (int)H, n, "fft_x_fwd_phi1", 2 * S);
+  DstPhi1<T> d{phi, (long long)n * H, n, (int)H, scale, 2.0 * M_PI / boxlen, amp, nn};
+  launch_col<T, false>(c, n, SrcPlain<T>{cd, 0, (long long)n * H}, d, (int)(n * H), 1, "fft_x_fwd_phi1", 2 * S);
 }
 
 template void fft_r2c_phi1<float>(Ctx&, float*, int, float, cx<float>*, double, const double*, NoiseNorm);
@@ -78,17 +89,32 @@ template void fft_r2c_phi1<double>(Ctx&, double*, int, double, cx<double>*, doub
 template <typename T>
 void fft_c2r_particles(Ctx& c, T* data, int n, T scale, double* out, int idim, double lunit, int kind,
                        const T* src, double qshift) {
+  double* const outs[1] = {out};
+  const int codes[1] = {idim | kind << 2};
+  fft_c2r_particle_set<T>(c, data, n, scale, 1, outs, codes, lunit, src, qshift);
+}
+
+// the same for `cnt` <= 6 grids, one after another in memory, one launch a pass
+template <typename T>
+void fft_c2r_particle_set(Ctx& c, T* data, int n, T scale, int cnt, double* const* out, const int* codes,
+                          double lunit, const T* src, double qshift) {
   MFX_REQUIRE(n % 2 == 0, "c2r requires an even last dimension");
+  MFX_REQUIRE(cnt >= 1 && cnt <= 6, "one to six components");
   const long long H = n / 2 + 1;
   cx<T>* cd = reinterpret_cast<cx<T>*>(data);
   const cx<T>* cs = src ? reinterpret_cast<const cx<T>*>(src) : cd;
-  const double S = (double)n * n * (n + 2) * sizeof(T);
-  launch_col<T, true>(c, n, SrcPlain<T>{cs, H, (long long)n * H}, DstPlain<T>{cd, H, (long long)n * H, T(1)},
-                      (int)H, n, "fft_x_inv", 2 * S);
+  const double S = (double)cnt * n * n * (n + 2) * sizeof(T);
+  PartOut po{};
+  for (int w = 0; w < cnt; ++w) {
+    po.out[w] = out[w];
+    po.codes |= (unsigned)codes[w] << (4 * w);
+  }
+  launch_x<T, true>(c, n, cs, cd, n * H, T(1), cnt, "fft_x_inv", 2 * S);
   launch_col<T, true>(c, n, SrcPlain<T>{cd, (long long)n * H, H}, DstPlain<T>{cd, (long long)n * H, H, T(1)},
-                      (int)H, n, "fft_y_inv", 2 * S);
-  launch_row_c2r_part<T>(c, n / 2, cd, H, (int)H, out, (long long)n * n, scale, idim, lunit, kind,
-                         qshift / (double)n * lunit, "fft_z_c2r_part", S + (double)n * n * n * sizeof(double));
+                      (int)H, cnt * n, "fft_y_inv", 2 * S);
+  launch_row_c2r_part<T>(c, n / 2, cd, H, (int)H, po, (long long)cnt * n * n, scale, lunit,
+                         qshift / (double)n * lunit, "fft_z_c2r_part",
+                         S + (double)cnt * n * n * n * sizeof(double));
 }
 
 // one column pass over plain strided lines (element (b, col, pos) at
@@ -110,6 +136,10 @@ template void col_pass_plain<double, true>(Ctx&, int, const cx<double>*, cx<doub
                                            int, double, const char*, double);
 template void fft_c2r_particles<float>(Ctx&, float*, int, float, double*, int, double, int, const float*, double);
 template void fft_c2r_particles<double>(Ctx&, double*, int, double, double*, int, double, int, const double*, double);
+template void fft_c2r_particle_set<float>(Ctx&, float*, int, float, int, double* const*, const int*, double,
+                                          const float*, double);
+template void fft_c2r_particle_set<double>(Ctx&, double*, int, double, int, double* const*, const int*, double,
+                                           const double*, double);
 template void fft_r2c_3d<float>(Ctx&, float*, int, int, int, float);
 template void fft_r2c_3d<double>(Ctx&, double*, int, int, int, double);
 template void fft_c2r_3d<float>(Ctx&, float*, int, int, int, float);
@@ -164,7 +194,7 @@ void conv2(Ctx& c, const cx<T>* fa, const MultSpec& ma, const cx<T>* fb, const M
   launch_col<T, false>(c, m, SrcPlain<T>{T2a, (long long)m * hp, hp}, DstTrunc<T>{T1a, (long long)n * hp, hp, n}, h,
                        m, "conv_p4_yfwd", bT2 + bT1);
   // P5: x-forward truncation + op into out [i][j][kz]
-  DstTruncOp<T> d5{out, HN, (long long)n * HN, n, op, T(opfac), s_out, 0, kfac};
+  DstTruncOp<T> d5{{out}, n, HN, (long long)n * HN, n, op, T(opfac), s_out, 0, kfac};
   launch_col<T, false>(c, m, SrcPlain<T>{T1a, hp, (long long)n * hp}, d5, h, n, "conv_p5_xfwd",
                        bT1 + (op == OP_ASSIGN ? bN : 2 * bN));
 }
@@ -243,13 +273,13 @@ void autotune_columns(Ctx& c, int L) {
       // a plain pass, so they are tuned on their own
       if (L % 3 == 0 && (L / 3) % 2 == 0) {
         const int nn = 2 * L / 3;
-        const TurnArgs<T> ta{buf, sb, sp, nn, T(1), T(1), buf, sb, sp};
+        const TurnArgs<T> ta{buf, sb, sp, nn, T(1), T(1), buf, sb, sp, nb, 0, 0};
         tune(COL_TURN, cls, true, [&] { launch_turn<T>(c, L, ta, ncols, nb, "tune", 0); });
         // the truncating forward pass with an output operator (the last x
         // pass of a convolution or LPT source), in place: each workgroup
         // writes only the retained positions of the lines it has read; these
         // passes always run plan 0
-        DstTruncOp<T> dt{buf, sb, sp, nn, OP_ASSIGN, T(0), T(1), 1, T(1)};
+        DstTruncOp<T> dt{{buf}, nb, sb, sp, nn, OP_ASSIGN, T(0), T(1), 1, T(1)};
         tune(COL_TRUNC_OP, cls, false,
              [&] { launch_col<T, false>(c, L, SrcPlain<T>{buf, sb, sp}, dt, ncols, nb, "tune", 0); });
       }

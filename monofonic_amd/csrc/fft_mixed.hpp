@@ -399,7 +399,7 @@ __global__ void __launch_bounds__(1024)
   const bool act = col < ncols;
   const int colc = act ? col : ncols - 1;
   lcx<T>* const ltw = lds_table(lt);
-  const cx<T>* const src = a.src + (long long)b * a.sb + colc;
+  const cx<T>* const src = a.from(b) + colc;
   mix_first<T, false>(
       x + c, C, p, t, nthr, ltw, [&](int n) { return src[(long long)n * a.sp]; },
       [&] { mix_copy_table(lt, tw, p.L); });
@@ -415,7 +415,7 @@ __global__ void __launch_bounds__(1024)
   }
   __syncthreads();
   mix_stages<T, true, true>(x + c, C, p, 1, p.nr - 1, t, nthr, ltw);
-  cx<T>* const out = a.out + (long long)b * a.osb + col;
+  cx<T>* const out = a.to(b) + col;
   auto done = [&](cx<T>* v, int k, int K, auto r) {
     constexpr int R = decltype(r)::value;
     if (act) {
@@ -577,19 +577,22 @@ __global__ void __launch_bounds__(512)
     }
 }
 
-// c2r writing FP64 particles (see k_row_c2r_part)
+// c2r writing FP64 particles (see k_row_c2r_part); n is even, so both rows of a
+// pair belong to one component
 template <typename T>
 __global__ void __launch_bounds__(512)
-    k_mix_c2r_part(const cx<T>* src, long long spitch, int hin, double* out, T scale, int idim, double lunit, int kind,
-                   double qoff, MixRowArgs a, const cx<T>* __restrict__ tw) {
+    k_mix_c2r_part(const cx<T>* src, long long spitch, int hin, PartOut po, T scale, double lunit, double qoff,
+                   MixRowArgs a, const cx<T>* __restrict__ tw) {
   extern __shared__ __align__(16) unsigned char col_lds_raw[];
   const MixRow<T> r(a, reinterpret_cast<cx<T>*>(col_lds_raw));
   const int n = a.p.L;
+  const int w = (int)(r.ra / ((long long)n * n)), code = po.code(w), idim = code & 3, kind = code >> 2;
   auto qrow = [&](long long row) {
-    return (double)(idim == 0 ? (int)(row / n) : (int)(row % n)) / (double)n * lunit + qoff;
+    return (double)(idim == 0 ? (int)(row / n) - w * n : (int)(row % n)) / (double)n * lunit + qoff;
   };
   const double qa = qrow(r.ra), qb = qrow(r.rb);
-  double *oa = out + r.ra * n, *ob = out + r.rb * n;
+  double* const o = po.array(w) - (long long)w * n * n * n;
+  double *oa = o + r.ra * n, *ob = o + r.rb * n;
   mix_c2r_rows<T>(r, a.p, src + r.ra * spitch, src + r.rb * spitch, hin, tw, [&](cx<T> v, int k) {
     double fa = (double)(v.x * scale), fb = (double)(v.y * scale);
     if (kind == 0) {

@@ -88,6 +88,19 @@ struct SrcPlain {
   }
 };
 
+// lines of several equal arrays in one launch: batch b is line set b % nb of
+// array b / nb, the arrays sq apart
+template <typename T>
+struct SrcSplit {
+  const cx<T>* p;
+  long long sb, sp, sq;
+  int nb;
+  __device__ __forceinline__ cx<T> load(int b, int col, int pos) const {
+    const int q = b / nb;
+    return p[(long long)q * sq + (long long)(b - q * nb) * sb + (long long)pos * sp + col];
+  }
+};
+
 template <typename T>
 struct DstPlain {
   cx<T>* p;
@@ -141,6 +154,37 @@ struct SrcPadPow {
   }
 };
 
+// The y stage of a field's Hessian rows in one launch: batch b is output b % 6
+// of x-plane b / 6.  Outputs 0..2 are the powers 0, 1, 2 of g_y of X_0, 3 and 4
+// the powers 0, 1 of X_1, 5 is X_2.  The outputs of a plane that share their
+// source follow one another on an XCD, a plane (1.1 MB at n = 512, FP32) apart,
+// so its second and third reads are served by that XCD's L2; six launches for a
+// field read it from HBM six times (Y_FIGURES).
+template <typename T>
+struct SrcHessY {
+  const cx<T>* x[3];
+  long long sb, sp;
+  int n;
+  T kfac;
+  __device__ __forceinline__ cx<T> load(int b, int col, int pos) const {
+    const int plane = b / 6, o = b - 6 * plane;
+    const cx<T>* p = o < 3 ? x[0] : (o < 5 ? x[1] : x[2]);
+    const int pw = o < 3 ? o : (o == 4 ? 1 : 0);
+    return SrcPadPow<T>{p, sb, sp, n, pw, T(1), kfac}.load(plane, col, pos);
+  }
+};
+template <typename T>
+struct DstHessY {
+  cx<T>* y[6];
+  long long sb, sp;
+  __device__ __forceinline__ cx<T> load_old(int, int, int) const { return mk(T(0), T(0)); }
+  __device__ __forceinline__ void store(int b, int col, int pos, cx<T> v, cx<T>) const {
+    const int plane = b / 6, o = b - 6 * plane;
+    cx<T>* p = o < 2 ? (o == 0 ? y[0] : y[1]) : (o < 4 ? (o == 2 ? y[2] : y[3]) : (o == 4 ? y[4] : y[5]));
+    p[(long long)plane * sb + (long long)pos * sp + col] = v;
+  }
+};
+
 // keep the n retained outputs of an M-line (convolution.hh:629-634)
 template <typename T>
 struct DstTrunc {
@@ -165,13 +209,17 @@ struct DstTrunc {
 // and the output operator on the flat k-space array (operators.hh:25-35)
 template <typename T>
 struct DstTruncOp {
-  cx<T>* out;
-  long long sb, sp;  // b = j stride, pos = i stride (complex units)
+  cx<T>* out[4];     // batch b is line set b % nb of output array b / nb
+  int nb;
+  long long sb, sp;  // line set (j) stride, pos (i) stride (complex units)
   int n;
   int op;
   T opfac, scale;
   int invlap;  // fold apply_InverseLaplacian (grid_fft.hh:440-449)
   T kfac;
+  __device__ __forceinline__ cx<T>* array(int q) const {
+    return q < 2 ? (q == 0 ? out[0] : out[1]) : (q == 2 ? out[2] : out[3]);
+  }
   // previous output value for the accumulating operators, loaded for every
   // element of the thread before any store (clamped index, no branch)
   __device__ __forceinline__ cx<T> load_old(int b, int col, int pos) const {
@@ -179,9 +227,10 @@ struct DstTruncOp {
     const int nh = n >> 1;
     const bool drop = (pos > nh) & (pos <= n);
     const int i = drop ? 0 : (pos <= nh ? pos : pos - nh);
-    return out[(long long)i * sp + (long long)b * sb + col];
+    const int q = b / nb;
+    return array(q)[(long long)i * sp + (long long)(b - q * nb) * sb + col];
   }
-  // output value at retained index i of line b, column col
+  // output value at retained index i of line set b, column col
   __device__ __forceinline__ cx<T> value(int b, int col, int i, cx<T> v, cx<T> prev) const {
     const int nh = n >> 1;
     const bool nyq = (i == nh) | (b == nh) | (col == nh);
@@ -211,7 +260,8 @@ struct DstTruncOp {
       i = pos - nh;
     else
       return;
-    out[(long long)i * sp + (long long)b * sb + col] = value(b, col, i, v, prev);
+    const int q = b / nb, j = b - q * nb;
+    array(q)[(long long)i * sp + (long long)j * sb + col] = value(j, col, i, v, prev);
   }
 };
 
@@ -220,19 +270,20 @@ struct DstTruncOp {
 // value is scaled as the plain pass would store it (rounded to T) and turned
 // into phi(1) by the same per-mode function the phi(1) kernel uses, so the
 // result is bit-identical to transform-then-phi(1).  Lines along x (pos = i),
-// batch j, column kz.
+// column j H + kz.
 template <typename T>
 struct DstPhi1 {
   cx<T>* phi;
-  long long sb, sp;
-  int n;
+  long long sp;
+  int n, H;
   T scale;
   double kfac;
   const double* amp;
   NoiseNorm nn;
   __device__ __forceinline__ cx<T> load_old(int, int, int) const { return mk(T(0), T(0)); }
-  __device__ __forceinline__ void store(int b, int col, int pos, cx<T> v, cx<T>) const {
-    phi[(long long)b * sb + (long long)pos * sp + col] = phi1_value(v * scale, pos, b, col, n, kfac, amp, nn);
+  __device__ __forceinline__ void store(int, int col, int pos, cx<T> v, cx<T>) const {
+    const int j = col / H;
+    phi[(long long)pos * sp + col] = phi1_value(v * scale, pos, j, col - j * H, n, kfac, amp, nn);
   }
 };
 
@@ -446,6 +497,16 @@ struct TurnArgs {
   T fscale, iscale;
   cx<T>* out;
   long long osb, osp;
+  int nb;            // line sets of one array; further arrays sq apart
+  long long sq, osq;
+  __device__ __forceinline__ const cx<T>* from(int b) const {
+    const int q = b / nb;
+    return src + (long long)q * sq + (long long)(b - q * nb) * sb;
+  }
+  __device__ __forceinline__ cx<T>* to(int b) const {
+    const int q = b / nb;
+    return out + (long long)q * osq + (long long)(b - q * nb) * osb;
+  }
 };
 
 template <typename T, int L, int C, int V = 0>
@@ -462,9 +523,10 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
   const bool act = col < ncols;
   const int colc = act ? col : ncols - 1;
   const int nh = a.n >> 1;
+  const cx<T>* const from = a.from(b);
   cx<T> x[EPT];
 #pragma unroll
-  for (int e = 0; e < EPT; ++e) x[e] = a.src[(long long)b * a.sb + (long long)(t + TPS * e) * a.sp + colc];
+  for (int e = 0; e < EPT; ++e) x[e] = from[(long long)(t + TPS * e) * a.sp + colc];
   const ColTw<T, L, C, V> ft(tw, twl);
   ft.template exec<false>(x, lds + c, C, t);
   const bool nyqc = colc == nh;
@@ -479,8 +541,9 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
   __syncthreads();  // the forward transform's exchange reads are done
   ft.template exec<true>(x, lds + c, C, t);
   if (act) {
+    cx<T>* const to = a.to(b);
 #pragma unroll
-    for (int e = 0; e < EPT; ++e) a.out[(long long)b * a.osb + (long long)(t + TPS * e) * a.osp + col] = x[e];
+    for (int e = 0; e < EPT; ++e) to[(long long)(t + TPS * e) * a.osp + col] = x[e];
   }
 }
 
@@ -501,8 +564,9 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
   auto fetch = [&](long long item, int tq, cx<T>(&v)[EPT]) {
     const int b = (int)(item / ntiles), col = (int)(item % ntiles) * C + c;
     const int colc = col < ncols ? col : ncols - 1;
+    const cx<T>* const from = a.from(b);
 #pragma unroll
-    for (int e = 0; e < EPT; ++e) v[e] = a.src[(long long)b * a.sb + (long long)(tq + TPS * e) * a.sp + colc];
+    for (int e = 0; e < EPT; ++e) v[e] = from[(long long)(tq + TPS * e) * a.sp + colc];
   };
   fetch(w, t, nx);
   const ColTw<T, L, C, V> ft(tw, twl);
@@ -527,8 +591,9 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
     __syncthreads();  // the forward transform's exchange reads are done
     ft.template exec<true>(x, lds + c, C, t);
     if (col < ncols) {
+      cx<T>* const to = a.to(b);
 #pragma unroll
-      for (int e = 0; e < EPT; ++e) a.out[(long long)b * a.osb + (long long)(tq + TPS * e) * a.osp + col] = x[e];
+      for (int e = 0; e < EPT; ++e) to[(long long)(tq + TPS * e) * a.osp + col] = x[e];
     }
   }
 }
@@ -693,6 +758,18 @@ inline bool col_plan_alt(int L) {
   }
 }
 
+// The particle arrays of up to six components of an n^3 grid, n^2 rows each, in
+// one launch: component w = row / n^2 goes to out[w]; code(w) & 3 is its axis,
+// code(w) >> 2 its kind (0 positions, 1 velocities).
+struct PartOut {
+  double* out[6];
+  unsigned codes;  // four bits for each component
+  __device__ __forceinline__ double* array(int w) const {
+    return w < 2 ? (w == 0 ? out[0] : out[1]) : (w < 4 ? (w == 2 ? out[2] : out[3]) : (w == 4 ? out[4] : out[5]));
+  }
+  __device__ __forceinline__ int code(int w) const { return (int)(codes >> (4 * w)) & 15; }
+};
+
 // ------------------------------------------------------------------ lengths without tuned kernels
 // (mixed_kernels.hip: run-time schedules)
 template <typename T, bool INV, class Src, class Dst>
@@ -706,8 +783,8 @@ template <typename T>
 void launch_row_c2r_any(Ctx& c, int K, const cx<T>* src, long long spitch, int hin, T* dst, long long dpitch,
                         long long nrows, T scale, const char* name, double bytes);
 template <typename T>
-void launch_row_c2r_part_any(Ctx& c, int K, const cx<T>* src, long long spitch, int hin, double* out, long long nrows,
-                             T scale, int idim, double lunit, int kind, double qoff, const char* name, double bytes);
+void launch_row_c2r_part_any(Ctx& c, int K, const cx<T>* src, long long spitch, int hin, const PartOut& po,
+                             long long nrows, T scale, double lunit, double qoff, const char* name, double bytes);
 template <typename T>
 void launch_row_prod_any(Ctx& c, int K, const cx<T>* a, const cx<T>* b, long long spitch, int hin, cx<T>* dst,
                          long long dpitch, int hout, long long nrows, const char* name, double bytes);
@@ -991,16 +1068,18 @@ __global__ void __launch_bounds__(RowLanes<K>::THREADS)
 // q_d = i_d/n * lunit.  Row r = i*n + j holds particles r*n .. r*n + n-1.
 template <typename T, int K>
 __global__ void __launch_bounds__(RowLanes<K>::THREADS)
-    k_row_c2r_part(const cx<T>* src, long long spitch, int hin, double* out, long long nrows, T scale, int idim,
-                   double lunit, int kind, double qoff, const cx<T>* __restrict__ twK, const cx<T>* __restrict__ twM) {
+    k_row_c2r_part(const cx<T>* src, long long spitch, int hin, PartOut po, long long nrows, T scale, double lunit,
+                   double qoff, const cx<T>* __restrict__ twK, const cx<T>* __restrict__ twM) {
   MFX_ROW_PROLOGUE(T, K)
   constexpr int E = RowCtx<T, K>::E, n = 2 * K;
   cx<T> v[E];
   rc.c2r(v, src + rowc * spitch, hin);
-  const int i = (int)(rowc / n), j = (int)(rowc % n);
+  const int rw = (int)(rowc / n);  // component w, x index i
+  const int w = rw / n, i = rw - w * n, j = (int)(rowc - (long long)rw * n);
+  const int code = po.code(w), idim = code & 3, kind = code >> 2;
   const double qrow = (double)(idim == 0 ? i : j) / (double)n * lunit + qoff;
-  const __amdgpu_buffer_rsrc_t r =
-      row_rsrc_u<RowLanes<K>::RPW == 1>(out + rowc * n, act ? (unsigned)(n * sizeof(double)) : 0u);
+  const __amdgpu_buffer_rsrc_t r = row_rsrc_u<RowLanes<K>::RPW == 1>(po.array(w) + ((long long)i * n + j) * n,
+                                                                     act ? (unsigned)(n * sizeof(double)) : 0u);
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     const int m = lane + P_ * e;
@@ -1113,24 +1192,24 @@ void launch_row_c2r(Ctx& c, int K, const cx<T>* src, long long spitch, int hin, 
 }
 
 template <typename T, int K>
-void launch_row_c2r_part_K(Ctx& c, const cx<T>* src, long long spitch, int hin, double* out, long long nrows, T scale,
-                           int idim, double lunit, int kind, double qoff, const char* name, double bytes) {
+void launch_row_c2r_part_K(Ctx& c, const cx<T>* src, long long spitch, int hin, const PartOut& po, long long nrows,
+                           T scale, double lunit, double qoff, const char* name, double bytes) {
   const dim3 grid = row_grid<T, K>(nrows);
   LaunchScope ls(c, name, bytes);
-  hipLaunchKernelGGL((k_row_c2r_part<T, K>), grid, dim3(RowBlk<T, K>::THREADS), 0, c.stream, src, spitch, hin, out, nrows, scale, idim,
-                     lunit, kind, qoff, c.twiddles<T>(K), c.twiddles<T>(2 * K));
+  hipLaunchKernelGGL((k_row_c2r_part<T, K>), grid, dim3(RowBlk<T, K>::THREADS), 0, c.stream, src, spitch, hin, po,
+                     nrows, scale, lunit, qoff, c.twiddles<T>(K), c.twiddles<T>(2 * K));
   check_launch(name);
 }
 
 template <typename T>
-void launch_row_c2r_part(Ctx& c, int K, const cx<T>* src, long long spitch, int hin, double* out, long long nrows,
-                         T scale, int idim, double lunit, int kind, double qoff, const char* name, double bytes) {
-#define MFX_CASE(KK)                                                                                            \
-  case KK:                                                                                                      \
-    launch_row_c2r_part_K<T, KK>(c, src, spitch, hin, out, nrows, scale, idim, lunit, kind, qoff, name, bytes); \
+void launch_row_c2r_part(Ctx& c, int K, const cx<T>* src, long long spitch, int hin, const PartOut& po,
+                         long long nrows, T scale, double lunit, double qoff, const char* name, double bytes) {
+#define MFX_CASE(KK)                                                                                  \
+  case KK:                                                                                            \
+    launch_row_c2r_part_K<T, KK>(c, src, spitch, hin, po, nrows, scale, lunit, qoff, name, bytes);    \
     return;
   MFX_ROW_SWITCH(K, MFX_CASE,
-                 launch_row_c2r_part_any<T>(c, K, src, spitch, hin, out, nrows, scale, idim, lunit, kind, qoff, name, bytes))
+                 launch_row_c2r_part_any<T>(c, K, src, spitch, hin, po, nrows, scale, lunit, qoff, name, bytes))
 #undef MFX_CASE
 }
 

@@ -548,8 +548,8 @@ struct Engine {
     bR = cs * (double)l.treal;
   }
 
-  // x and y stages of a field: Hessian rows (six Y arrays) or one plain Y0
-  void inverse(const cx<T>* F, bool hessian, cx<T>* const* Y) {
+  // x and y stages of a field: its Hessian rows into the six arrays at Y
+  void inverse(const cx<T>* F, cx<T>* const* Y) {
     const int n = l.n, m = l.m, hp = l.hp;
     const long long HN = l.h;
     // x stage: line along i of the n-grid [i][j][kz], batch j, output [x][j][kz]:
@@ -559,59 +559,61 @@ struct Engine {
                   DstPlain<T>{nullptr, hp, (long long)n * hp, T(1)},
                   {T1[0], T1[1], T1[2]},
                   {0, 1, 2},
-                  hessian ? 3 : 1};
+                  3};
     launch_col_multi<T, true>(c, m, a, l.h, n, "lpt_x_inv", bN, bT1);
-    y_inverse(hessian, Y);
+    // y stage: line along j of T1 [x][j][kz], output [x][y][kz]: Y0, Yy, Yyy
+    // from X_0, Yx, Yxy from X_1, Yxx from X_2
+    SrcHessY<T> s{{T1[0], T1[1], T1[2]}, (long long)n * hp, hp, n, kfac};
+    DstHessY<T> d{{Y[0], Y[2], Y[5], Y[1], Y[4], Y[3]}, (long long)m * hp, hp};
+    launch_col_pad<T, true>(c, m, s, d, l.h, 6 * m, "lpt_y_inv", 3 * bT1 + 6 * bT2);
   }
 
-  // y stage: line along j of T1 [x][j][kz], batch x, output [x][y][kz]; one
-  // launch per output (a multi-output launch that re-reads its source tile
-  // from the L2 measured slower here than separate launches: 6.2 vs 5.8 ms
-  // for the twelve 768-line outputs of 3LPT at 512^3)
-  void y_inverse(bool hessian, cx<T>* const* Y) {
+  // How many of `cnt` equal arrays of `bytes` go through a chain of passes in one
+  // launch each: all of them where they fit the 256 MiB memory-side cache with
+  // room to spare (a chain's next pass then still finds them there, and a small
+  // grid's launches, whose 4 to 15 us hardly depend on the work, are fewer), one at
+  // a time where a single array does not (LPT_FIGURES).
+  static int together(int cnt, double bytes) {
+    const int fit = (int)(160.0 * (1 << 20) / bytes);
+    const int groups = fit < 1 ? cnt : (cnt + fit - 1) / fit;
+    return (cnt + groups - 1) / groups;
+  }
+
+  // y and x forward transforms of the z-stage outputs in `cnt` adjacent y/z slots
+  // at Z into n-grids, through the x-stage slots at work (cnt of them)
+  void forward(cx<T>* Z, int cnt, cx<T>* work, cx<T>* const* out, bool invlap) {
     const int n = l.n, m = l.m, hp = l.hp;
-    auto ystage = [&](int src, std::initializer_list<std::pair<int, int>> outs) {
-      for (auto& o : outs)
-        launch_col_pad<T, true>(c, m, SrcPadPow<T>{T1[src], (long long)n * hp, hp, n, o.second, T(1), kfac},
-                                DstPlain<T>{Y[o.first], (long long)m * hp, hp, T(1)}, l.h, m, "lpt_y_inv", bT1 + bT2);
-    };
-    if (hessian) {
-      ystage(0, {{0, 0}, {2, 1}, {5, 2}});  // Y0, Yy, Yyy
-      ystage(1, {{1, 0}, {4, 1}});          // Yx, Yxy
-      ystage(2, {{3, 0}});                  // Yxx
-    } else {
-      ystage(0, {{0, 0}});
+    const long long HN = l.h;
+    const int g = together(cnt, bT1);
+    for (int q = 0; q < cnt; q += g) {
+      const int k = q + g < cnt ? g : cnt - q;
+      launch_col_pad<T, false>(c, m, SrcPlain<T>{Z + q * l.t2, (long long)m * hp, hp},
+                               DstTrunc<T>{work, (long long)n * hp, hp, n}, l.h, k * m, "lpt_y_fwd", k * (bT2 + bT1));
+      DstTruncOp<T> d{{}, n, HN, (long long)n * HN, n, OP_ASSIGN, T(0), s_out, invlap ? 1 : 0, kfac};
+      for (int i = 0; i < k; ++i) d.out[i] = out[q + i];
+      launch_col_pad<T, false>(c, m, SrcSplit<T>{work, hp, (long long)n * hp, (long long)l.t1, n}, d, l.h, k * n,
+                               "lpt_x_fwd", k * (bT1 + bN));
     }
   }
 
-  // y forward of a z-stage output into T1[0] (the n retained rows)
-  void y_forward(cx<T>* Z) {
+  // the 3a intermediates of OrszagConvolver::convolve3: `cnt` adjacent z-stage
+  // outputs at Z truncated to the n-grid and padded back into the slots at Y
+  // (which may be Z), without the n-grid fields.  The truncation (with its
+  // Nyquist zeroing) is a separable projection, so it runs as one y pass over
+  // the M x-planes of a slot (Z into Y) and one x pass over its M y rows (Y in
+  // place, with the Orszag scales sqrt(n^3)/M^3 and 1/sqrt(n^3)).
+  void turn(const cx<T>* Z, cx<T>* Y, int cnt) {
     const int n = l.n, m = l.m, hp = l.hp;
-    launch_col_pad<T, false>(c, m, SrcPlain<T>{Z, (long long)m * hp, hp}, DstTrunc<T>{T1[0], (long long)n * hp, hp, n},
-                             l.h, m, "lpt_y_fwd", bT2 + bT1);
-  }
-
-  // y and x forward transforms of a z-stage output into an n-grid
-  void forward(cx<T>* Z, cx<T>* out, bool invlap) {
-    const int n = l.n, m = l.m, hp = l.hp;
-    const long long HN = l.h;
-    y_forward(Z);
-    DstTruncOp<T> d{out, HN, (long long)n * HN, n, OP_ASSIGN, T(0), s_out, invlap ? 1 : 0, kfac};
-    launch_col_pad<T, false>(c, m, SrcPlain<T>{T1[0], hp, (long long)n * hp}, d, l.h, n, "lpt_x_fwd", bT1 + bN);
-  }
-
-  // the 3a intermediates of OrszagConvolver::convolve3: a z-stage output
-  // truncated to the n-grid and padded back, without the n-grid field.  The
-  // truncation (with its Nyquist zeroing) is a separable projection, so it
-  // runs as one y pass over the M x-planes of the slot (Z into Y) and one x
-  // pass over its M y rows (Y in place, with the Orszag scales sqrt(n^3)/M^3
-  // and 1/sqrt(n^3)).
-  void turn(cx<T>* Z, cx<T>* Y) {
-    const int n = l.n, m = l.m, hp = l.hp;
-    TurnArgs<T> ay{Z, (long long)m * hp, hp, n, T(1), T(1), Y, (long long)m * hp, hp};
-    launch_turn<T>(c, m, ay, l.h, m, "lpt_y_turn", 2 * bT2);
-    TurnArgs<T> ax{Y, hp, (long long)m * hp, n, s_out, s_in, Y, hp, (long long)m * hp};
-    launch_turn<T>(c, m, ax, l.h, m, "lpt_x_turn", 2 * bT2);
+    const long long t2 = (long long)l.t2, mh = (long long)m * hp;
+    const int g = together(cnt, bT2);
+    for (int q = 0; q < cnt; q += g) {
+      const int k = q + g < cnt ? g : cnt - q;
+      cx<T>* y = Y + q * t2;
+      TurnArgs<T> ay{Z + q * t2, mh, hp, n, T(1), T(1), y, mh, hp, m, t2, t2};
+      launch_turn<T>(c, m, ay, l.h, k * m, "lpt_y_turn", k * 2 * bT2);
+      TurnArgs<T> ax{y, hp, mh, n, s_out, s_in, y, hp, mh, m, t2, t2};
+      launch_turn<T>(c, m, ax, l.h, k * m, "lpt_x_turn", k * 2 * bT2);
+    }
   }
 
   FieldY<T> fy(int base) const {
@@ -631,7 +633,7 @@ void lpt_sources(Ctx& c, const cx<T>* phi, cx<T>* phi2, cx<T>* phi3, cx<T>* a3x,
   const long long nrows = (long long)l.m * l.m;
   const bool three = order > 2;
   // phi: Hessian rows into T2[0..5]
-  E.inverse(phi, true, E.T2);
+  E.inverse(phi, E.T2);
   const FieldY<T> fphi = E.fy(0);
   // stage A: S2 -> T2[6]; I1..I4 -> T2[7..10]
   cx<T>* Iz[4] = {E.T2[7], E.T2[8], E.T2[9], E.T2[10]};
@@ -646,44 +648,38 @@ void lpt_sources(Ctx& c, const cx<T>* phi, cx<T>* phi2, cx<T>* phi3, cx<T>* a3x,
                                      bytes))
 #undef MFX_CASE
   }
+  cx<T>* const phi2s[1] = {phi2};
   if (!three) {
-    E.forward(E.T2[6], phi2, true);  // phi2 = -S2/k^2 (ic_generator.cc:488)
+    E.forward(E.T2[6], 1, E.T1[0], phi2s, true);  // phi2 = -S2/k^2 (ic_generator.cc:488)
     return;
   }
   // the 3a intermediates go forward to the n-grid (truncation) and straight
   // back to their rows
-  auto turn_I = [&](int q, cx<T>* row) { E.turn(Iz[q], row); };
   if (E.R) {
     // stored: phi's Hessian rows are dead after stage A, so phi2's take
-    // T2[0..5], then intermediate q's row moves from T2[7+q] to T2[6+q]
-    E.forward(E.T2[6], phi2, true);  // phi2 = -S2/k^2 (ic_generator.cc:488)
-    E.inverse(phi2, true, E.T2);
-    cx<T>* Ir[4];
-    for (int q = 0; q < 4; ++q) {
-      Ir[q] = E.T2[6 + q];
-      turn_I(q, Ir[q]);
-    }
+    // T2[0..5]; after stage C those are free in turn
+    E.forward(E.T2[6], 1, E.T1[0], phi2s, true);  // phi2 = -S2/k^2 (ic_generator.cc:488)
+    E.inverse(phi2, E.T2);
+    E.turn(Iz[0], Iz[0], 4);
     const double bytes = 10 * E.bT2 + 6 * E.bR + 4 * E.bT2;
 #define MFX_CASE(KK)                                                                                   \
   case KK:                                                                                             \
-    launch_zC_K<T, KK>(c, E.fy(0), E.R, (long long)l.treal, Ir, l.hp, l.h, n, E.kfac, nrows, bytes); \
+    launch_zC_K<T, KK>(c, E.fy(0), E.R, (long long)l.treal, Iz, l.hp, l.h, n, E.kfac, nrows, bytes); \
     break;
     MFX_LPT_KSWITCH(K, MFX_CASE,
-                    launch_zC_mix<T>(c, E.fy(0), E.R, (long long)l.treal, Ir, l.hp, l.h, n, E.kfac, nrows, bytes))
+                    launch_zC_mix<T>(c, E.fy(0), E.R, (long long)l.treal, Iz, l.hp, l.h, n, E.kfac, nrows, bytes))
 #undef MFX_CASE
-    cx<T>* out[4] = {phi3, a3x, a3y, a3z};
-    for (int q = 0; q < 4; ++q) E.forward(Ir[q], out[q], true);
+    cx<T>* const out[4] = {phi3, a3x, a3y, a3z};
+    E.forward(Iz[0], 4, E.T2[0], out, true);
     return;
   }
-  // streamed: I1..I4 rows -> T2[12..15] first, then phi2's Hessian rows over
-  // S2 and the intermediates' z rows in T2[6..11]
+  // streamed: I1..I4 go to T2[12..15], then phi2's Hessian rows over S2 and
+  // the intermediates' z rows in T2[6..11]
   cx<T>* Ir[4];
-  for (int q = 0; q < 4; ++q) {
-    Ir[q] = E.T2[12 + q];
-    turn_I(q, Ir[q]);
-  }
-  E.forward(E.T2[6], phi2, true);
-  E.inverse(phi2, true, E.T2 + 6);
+  for (int q = 0; q < 4; ++q) Ir[q] = E.T2[12 + q];
+  E.turn(Iz[0], Ir[0], 4);
+  E.forward(E.T2[6], 1, E.T1[0], phi2s, true);
+  E.inverse(phi2, E.T2 + 6);
   const FieldY<T> fphi2 = E.fy(6);
   // stage C1: phi3 source over I1's rows
   {
@@ -695,7 +691,8 @@ void lpt_sources(Ctx& c, const cx<T>* phi, cx<T>* phi2, cx<T>* phi3, cx<T>* a3x,
     MFX_LPT_KSWITCH(K, MFX_CASE, MFX_LPT_NONE(K))
 #undef MFX_CASE
   }
-  E.forward(Ir[0], phi3, true);
+  cx<T>* const phi3s[1] = {phi3};
+  E.forward(Ir[0], 1, E.T1[0], phi3s, true);
   // stage C2: A3 components over I2..I4's rows
   cx<T>* A3[3] = {a3x, a3y, a3z};
   for (int i = 0; i < 3; ++i) {
@@ -706,7 +703,7 @@ void lpt_sources(Ctx& c, const cx<T>* phi, cx<T>* phi2, cx<T>* phi3, cx<T>* a3x,
     break;
     MFX_LPT_KSWITCH(K, MFX_CASE, MFX_LPT_NONE(K))
 #undef MFX_CASE
-    E.forward(Ir[1 + i], A3[i], true);
+    E.forward(Ir[1 + i], 1, E.T1[0], &A3[i], true);
   }
 }
 

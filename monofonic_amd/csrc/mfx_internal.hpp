@@ -142,6 +142,11 @@ void fft_c2r_3d(Ctx& c, T* data, int n0, int n1, int n2, T scale);
 template <typename T>
 void fft_c2r_particles(Ctx& c, T* data, int n, T scale, double* out, int idim, double lunit, int kind,
                        const T* src = nullptr, double qshift = 0.0);
+// cnt <= 6 grids one after another into the arrays out[0..cnt-1]; codes: axis |
+// kind << 2 of each
+template <typename T>
+void fft_c2r_particle_set(Ctx& c, T* data, int n, T scale, int cnt, double* const* out, const int* codes,
+                          double lunit, const T* src = nullptr, double qshift = 0.0);
 // one column pass over plain strided lines (element (b, col, pos) at
 // b*sb + pos*sp + col) from src to dst, the tuned kernel for length L
 template <typename T, bool INV>

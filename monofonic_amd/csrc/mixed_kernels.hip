@@ -236,7 +236,8 @@ MFX_COL_ANY(false, SrcPlain, DstTruncOp)
 MFX_COL_ANY(true, SrcPlain, DstPlain)
 MFX_COL_ANY(true, PadMult, DstPlain)
 MFX_COL_ANY(true, PadOnly, DstPlain)
-MFX_COL_ANY(true, SrcPadPow, DstPlain)
+MFX_COL_ANY(true, SrcHessY, DstHessY)
+MFX_COL_ANY(false, SrcSplit, DstTruncOp)
 MFX_COL_ANY(true, PowSrc, PowDst)
 #undef MFX_COL_ANY
 template void launch_turn_any<float>(Ctx&, int, const TurnArgs<float>&, int, int, const char*, double);
@@ -298,13 +299,13 @@ void launch_row_c2r_any(Ctx& c, int K, const cx<T>* src, long long spitch, int h
 }
 
 template <typename T>
-void launch_row_c2r_part_any(Ctx& c, int K, const cx<T>* src, long long spitch, int hin, double* out, long long nrows,
-                             T scale, int idim, double lunit, int kind, double qoff, const char* name, double bytes) {
+void launch_row_c2r_part_any(Ctx& c, int K, const cx<T>* src, long long spitch, int hin, const PartOut& po,
+                             long long nrows, T scale, double lunit, double qoff, const char* name, double bytes) {
   const MixCfg& m = mix_cfg<T>(c, 2 * K, MIX_ROW);
   if (m.ok)
-    MFX_MIX_ROW(k_mix_c2r_part, m, src, spitch, hin, out, scale, idim, lunit, kind, qoff);
+    MFX_MIX_ROW(k_mix_c2r_part, m, src, spitch, hin, po, scale, lunit, qoff);
   else
-    MFX_GEN_ROW(k_row_c2r_part_gen, 2, src, spitch, hin, out, scale, idim, lunit, kind, qoff);
+    MFX_GEN_ROW(k_row_c2r_part_gen, 2, src, spitch, hin, po, scale, lunit, qoff);
 }
 
 template <typename T>
@@ -322,8 +323,8 @@ void launch_row_prod_any(Ctx& c, int K, const cx<T>* a, const cx<T>* b, long lon
                                       const char*, double);                                                        \
   template void launch_row_c2r_any<T>(Ctx&, int, const cx<T>*, long long, int, T*, long long, long long, T,        \
                                       const char*, double);                                                        \
-  template void launch_row_c2r_part_any<T>(Ctx&, int, const cx<T>*, long long, int, double*, long long, T, int,    \
-                                           double, int, double, const char*, double);                              \
+  template void launch_row_c2r_part_any<T>(Ctx&, int, const cx<T>*, long long, int, const PartOut&, long long, T,  \
+                                           double, double, const char*, double);                                   \
   template void launch_row_prod_any<T>(Ctx&, int, const cx<T>*, const cx<T>*, long long, int, cx<T>*, long long,   \
                                        int, long long, const char*, double);
 MFX_ROW_ANY(float)
