@@ -180,18 +180,6 @@ template <typename T>
 __device__ __forceinline__ cx<T> ld(lcx<T>* p, int i) {
   return mk(p[i].x, p[i].y);
 }
-// An LDS table of the first H = L/2 twiddles only: w^(i + L/2) = -w^i
-template <typename T, int H>
-struct HalfTw {
-  lcx<T>* p;
-};
-template <typename T, int H>
-__device__ __forceinline__ cx<T> ld(HalfTw<T, H> h, int i) {
-  const bool up = i >= H;
-  const cx<T> v = ld(h.p, up ? i - H : i);
-  return up ? mk(-v.x, -v.y) : v;
-}
-
 // ---------------------------------------------------------------- plans
 // Radix schedule per length and variant V: EPT must be a multiple of every
 // radix.  Variant 0 exists for every length; some lengths have a variant 1
@@ -364,46 +352,52 @@ __device__ __forceinline__ void fft_exec(cx<T> (&v)[EPT], cx<T>* lds, int ls, in
   stage_loop<T, L, INV, 0, V>(v, lds, ls, t, global_table(tw), w0);
 }
 
-// fft_exec with the twiddle table copied to LDS at twl (L entries, or the
-// first L/2 with HALF; visible to every thread: the copy is followed by a
-// barrier before the first call)
-template <typename T, int L, bool INV, int V = 0, bool HALF = false, int EPT>
+// fft_exec with the twiddle table copied to LDS at twl (TwCount entries,
+// visible to every thread: the copy is followed by a barrier before the first
+// call)
+template <typename T, int L, bool INV, int V = 0, int EPT>
 __device__ __forceinline__ void fft_exec_lt(cx<T> (&v)[EPT], cx<T>* lds, int ls, int t, const cx<T>* twl) {
   static_assert(EPT == Plan<L, V>::EPT, "register array of the plan");
-  if constexpr (HALF)
-    stage_loop_lt<T, L, INV, 0, V>(v, lds, ls, t, HalfTw<T, L / 2>{lds_table(twl)});
-  else
-    stage_loop_lt<T, L, INV, 0, V>(v, lds, ls, t, lds_table(twl));
+  stage_loop_lt<T, L, INV, 0, V>(v, lds, ls, t, lds_table(twl));
 }
 
-// LDS layout of a column workgroup of C lines of length L, all in dynamic LDS:
-// the exchange area (L*C values) followed by the twiddle table.  Where a full
-// table would keep a third workgroup off a compute unit (160 KiB of LDS) and
-// half of it would not, only the first L/2 twiddles are kept (HalfTw): e.g.
-// 768-line FP32 tiles of 8 columns, 51 instead of 54 KiB per workgroup, three
-// workgroups per CU instead of two.
-template <typename T, int L, int C>
+// twiddles that the plan's stages read: w^i for i up to (R - 1)(NS - 1) L/(NS R)
+template <int L, int V>
+constexpr int tw_count() {
+  int most = 0, ns = 1;
+  for (int s = 0; s < Plan<L, V>::NR; ++s) {
+    const int R = Plan<L, V>::R[s], i = (R - 1) * (ns - 1) * (L / (ns * R));
+    if (i > most) most = i;
+    ns *= R;
+  }
+  return most + 1;
+}
+
+// LDS layout of a column workgroup of C lines of length L (plan V), all in
+// dynamic LDS: the exchange area (L*C values) followed by the twiddles the plan
+// reads, at most 3/4 of the table after a first radix of 12.  768-line FP32 tiles of
+// 8 columns then take 52.5 KiB, three workgroups on a compute unit's 160 KiB; with
+// the whole table two fit, and with half of it (w^(i + L/2) = -w^i by selects) a
+// tenth of the kernel's instructions were those selects.
+template <typename T, int L, int C, int V>
 struct TwLds {
-  static constexpr long long cs = sizeof(cx<T>), cu = 160 * 1024;
-  static constexpr bool half = 3 * ((long long)L * C + L) * cs > cu && 3 * ((long long)L * C + L / 2) * cs <= cu;
-  static constexpr int entries = half ? L / 2 : L;
+  static constexpr int entries = tw_count<L, V>();
   static constexpr size_t bytes = (size_t)((long long)L * C + entries) * sizeof(cx<T>);
 };
 
-// Copies the twiddle table (its first TwLds::entries values) into LDS at lt
-// and runs the transforms through it.  Construct once per workgroup, before
-// any transform; the constructor ends with a barrier.
+// Copies the twiddles (TwLds::entries values) into LDS at lt and runs the
+// transforms through them.  Construct once per workgroup, before any transform;
+// the constructor ends with a barrier.
 template <typename T, int L, int C, int V>
 struct ColTw {
-  static constexpr bool HALF = TwLds<T, L, C>::half;
   cx<T>* s;
   __device__ __forceinline__ ColTw(const cx<T>* tw, cx<T>* lt) : s(lt) {
-    for (int i = threadIdx.x; i < TwLds<T, L, C>::entries; i += blockDim.x) s[i] = tw[i];
+    for (int i = threadIdx.x; i < TwLds<T, L, C, V>::entries; i += blockDim.x) s[i] = tw[i];
     __syncthreads();
   }
   template <bool INV, int EPT>
   __device__ __forceinline__ void exec(cx<T> (&v)[EPT], cx<T>* lds, int ls, int t) const {
-    fft_exec_lt<T, L, INV, V, HALF>(v, lds, ls, t, s);
+    fft_exec_lt<T, L, INV, V>(v, lds, ls, t, s);
   }
 };
 

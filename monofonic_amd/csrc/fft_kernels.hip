@@ -30,7 +30,7 @@ namespace mfx {
 // (j, kz) of a plane are adjacent, so they form one range of columns.  Tiles then
 // start at whole multiples of their width, on 128-byte lines where the plane
 // stride is one, and no row ends in a partial tile (at 512^3 a row of 257 columns
-// took 17 tiles of 16, each across two lines; X_FIGURES).
+// took 17 tiles of 16, each across two lines: 0.281 against 0.266 ms a pass).
 template <typename T, bool INV>
 static void launch_x(Ctx& c, int L, const cx<T>* src, cx<T>* dst, long long plane, T scale, int narr,
                      const char* name, double bytes) {

@@ -29,7 +29,7 @@ struct ColCfg {
   static constexpr int lim = (lim_lds < lim_thr ? lim_lds : lim_thr) < 16 ? (lim_lds < lim_thr ? lim_lds : lim_thr) : 16;
   static constexpr int C = lim >= 16 ? 16 : lim >= 8 ? 8 : lim >= 4 ? 4 : lim >= 2 ? 2 : 1;
   static constexpr int CW =
-      (C < 16 && 2 * C * TPS <= 1024 && TwLds<T, L, 2 * C>::bytes <= (size_t)160 * 1024) ? 2 * C : 0;
+      (C < 16 && 2 * C * TPS <= 1024 && TwLds<T, L, 2 * C, V>::bytes <= (size_t)160 * 1024) ? 2 * C : 0;
 };
 
 
@@ -79,12 +79,69 @@ MultDev<T> to_dev(const MultSpec& m) {
   return d;
 }
 
+// Position t + c of a line: in the tuned column kernels c = W e is the constant of
+// a thread's element e (W threads a line of L positions), so that a line's
+// address is formed once for each thread and an element adds a uniform stride,
+// and what depends on the range c .. c + W - 1 is decided when the kernel is
+// compiled.  From a plain position (the run-time kernels) W = 0.
+struct Pos {
+  int t, c, W, L;
+  __device__ __forceinline__ Pos(int p) : t(p), c(0), W(0), L(0) {}
+  __device__ __forceinline__ Pos(int t_, int c_, int W_, int L_) : t(t_), c(c_), W(W_), L(L_) {}
+  __device__ __forceinline__ operator int() const { return t + c; }
+};
+
+// element t + c of a line: column col of line set base (uniform), line stride sp
+template <typename C>
+__device__ __forceinline__ C* line_at(C* base, long long sp, int col, int t, int c) {
+  return base + ((long long)t * sp + col) + (long long)c * sp;
+}
+
+// Position of a line padded from n to 3n/2: kept positions hold index t + c of the
+// n-grid, whose signed wave index is t + k0 (n/2 positive); the others are zero.
+// drop(): no position of the element's range is kept.
+struct Kept {
+  bool keep, nyq;
+  int t, c, k0;
+  static __device__ __forceinline__ bool drop(const Pos& p) {
+    return p.W && p.c > p.L / 3 && p.c + p.W - 1 <= 2 * (p.L / 3);
+  }
+  __device__ __forceinline__ Kept(const Pos& p, int n) {
+    const int m = p.W ? 2 * (p.L / 3) : n, nh = m >> 1;
+    if (p.W && p.c + p.W - 1 < nh) {
+      keep = true;
+      nyq = false;
+      t = p.t;
+      c = k0 = p.c;
+    } else if (p.W && p.c == nh && p.c + p.W - 1 <= m) {
+      // the Nyquist position and padding: every lane addresses the former
+      keep = nyq = p.t == 0;
+      t = 0;
+      c = k0 = nh;
+    } else if (p.W && p.c >= m) {
+      keep = p.c > m || p.t != 0;
+      nyq = false;
+      t = p.t;
+      c = p.c - nh;
+      k0 = p.c - (m + nh);
+    } else {
+      const int q = p.t + p.c;
+      const bool pad = (q > nh) & (q <= m);
+      keep = !pad;
+      t = pad ? 0 : (q <= nh ? q : q - nh);
+      c = 0;
+      nyq = t == nh;
+      k0 = t > nh ? -m : 0;
+    }
+  }
+};
+
 template <typename T>
 struct SrcPlain {
   const cx<T>* p;
   long long sb, sp;
-  __device__ __forceinline__ cx<T> load(int b, int col, int pos) const {
-    return p[(long long)b * sb + (long long)pos * sp + col];
+  __device__ __forceinline__ cx<T> load(int b, int col, Pos pos) const {
+    return *line_at(p + (long long)b * sb, sp, col, pos.t, pos.c);
   }
 };
 
@@ -95,9 +152,9 @@ struct SrcSplit {
   const cx<T>* p;
   long long sb, sp, sq;
   int nb;
-  __device__ __forceinline__ cx<T> load(int b, int col, int pos) const {
+  __device__ __forceinline__ cx<T> load(int b, int col, Pos pos) const {
     const int q = b / nb;
-    return p[(long long)q * sq + (long long)(b - q * nb) * sb + (long long)pos * sp + col];
+    return *line_at(p + (long long)q * sq + (long long)(b - q * nb) * sb, sp, col, pos.t, pos.c);
   }
 };
 
@@ -107,8 +164,8 @@ struct DstPlain {
   long long sb, sp;
   T scale;
   __device__ __forceinline__ cx<T> load_old(int, int, int) const { return mk(T(0), T(0)); }
-  __device__ __forceinline__ void store(int b, int col, int pos, cx<T> v, cx<T>) const {
-    p[(long long)b * sb + (long long)pos * sp + col] = v * scale;
+  __device__ __forceinline__ void store(int b, int col, Pos pos, cx<T> v, cx<T>) const {
+    *line_at(p + (long long)b * sb, sp, col, pos.t, pos.c) = v * scale;
   }
 };
 
@@ -124,14 +181,13 @@ struct SrcPad {
   MultDev<T> m;  // used when MULT: line axis = x (i), b = y (j), col = kz
   // The load is unconditional (index clamped into the line) and the padding
   // is applied by a select, so all loads of a thread can be in flight at once.
-  __device__ __forceinline__ cx<T> load(int b, int col, int pos) const {
-    const int nh = n >> 1;
-    const bool pad = (pos > nh) & (pos <= n);
-    const int i = pad ? 0 : (pos <= nh ? pos : pos - nh);
-    cx<T> v = p[(long long)b * sb + (long long)i * sp + col];
-    if (MULT) v = cmul(v, m.eval(i, b, col, n, kfac));
+  __device__ __forceinline__ cx<T> load(int b, int col, Pos pos) const {
+    if (Kept::drop(pos)) return mk(T(0), T(0));
+    const Kept k(pos, n);
+    cx<T> v = *line_at(p + (long long)b * sb, sp, col, k.t, k.c);
+    if (MULT) v = cmul(v, m.eval(k.t + k.c, b, col, n, kfac));
     v = v * scale;
-    return pad ? mk(T(0), T(0)) : v;
+    return k.keep ? v : mk(T(0), T(0));
   }
 };
 
@@ -143,30 +199,30 @@ struct SrcPadPow {
   long long sb, sp;
   int n, pw;
   T scale, kfac;
-  __device__ __forceinline__ cx<T> load(int b, int col, int pos) const {
-    const int nh = n >> 1;
-    const bool pad = (pos > nh) & (pos <= n);
-    const int i = pad ? 0 : (pos <= nh ? pos : pos - nh);
-    const cx<T> x = p[(long long)b * sb + (long long)i * sp + col];
-    const T g = kval<T>(i, n, kfac, 1);
-    const T f = pw == 0 ? scale : (pw == 1 ? scale * g : scale * g * g);
-    return pad ? mk(T(0), T(0)) : x * f;
+  __device__ __forceinline__ cx<T> load(int b, int col, Pos pos) const {
+    if (Kept::drop(pos)) return mk(T(0), T(0));
+    const Kept k(pos, n);
+    const cx<T> x = *line_at(p + (long long)b * sb, sp, col, k.t, k.c);
+    const T g = k.nyq ? T(0) : T(k.t + k.k0) * kfac;
+    const T f1 = pw == 0 ? scale : scale * g;
+    const T f = pw == 2 ? f1 * g : f1;
+    return k.keep ? x * f : mk(T(0), T(0));
   }
 };
 
 // The y stage of a field's Hessian rows in one launch: batch b is output b % 6
 // of x-plane b / 6.  Outputs 0..2 are the powers 0, 1, 2 of g_y of X_0, 3 and 4
 // the powers 0, 1 of X_1, 5 is X_2.  The outputs of a plane that share their
-// source follow one another on an XCD, a plane (1.1 MB at n = 512, FP32) apart,
-// so its second and third reads are served by that XCD's L2; six launches for a
-// field read it from HBM six times (Y_FIGURES).
+// source follow one another on an XCD, a plane (1.1 MB at n = 512, FP32) apart.
+// One launch instead of six: 96^3 FP64 75 -> 47 us for a field, 256^3 FP64 0.82 ->
+// 0.67 ms, 512^3 FP32 2.80 -> 2.75 ms.
 template <typename T>
 struct SrcHessY {
   const cx<T>* x[3];
   long long sb, sp;
   int n;
   T kfac;
-  __device__ __forceinline__ cx<T> load(int b, int col, int pos) const {
+  __device__ __forceinline__ cx<T> load(int b, int col, Pos pos) const {
     const int plane = b / 6, o = b - 6 * plane;
     const cx<T>* p = o < 3 ? x[0] : (o < 5 ? x[1] : x[2]);
     const int pw = o < 3 ? o : (o == 4 ? 1 : 0);
@@ -178,10 +234,10 @@ struct DstHessY {
   cx<T>* y[6];
   long long sb, sp;
   __device__ __forceinline__ cx<T> load_old(int, int, int) const { return mk(T(0), T(0)); }
-  __device__ __forceinline__ void store(int b, int col, int pos, cx<T> v, cx<T>) const {
+  __device__ __forceinline__ void store(int b, int col, Pos pos, cx<T> v, cx<T>) const {
     const int plane = b / 6, o = b - 6 * plane;
     cx<T>* p = o < 2 ? (o == 0 ? y[0] : y[1]) : (o < 4 ? (o == 2 ? y[2] : y[3]) : (o == 4 ? y[4] : y[5]));
-    p[(long long)plane * sb + (long long)pos * sp + col] = v;
+    *line_at(p + (long long)plane * sb, sp, col, pos.t, pos.c) = v;
   }
 };
 
@@ -192,16 +248,10 @@ struct DstTrunc {
   long long sb, sp;
   int n;
   __device__ __forceinline__ cx<T> load_old(int, int, int) const { return mk(T(0), T(0)); }
-  __device__ __forceinline__ void store(int b, int col, int pos, cx<T> v, cx<T>) const {
-    const int nh = n >> 1;
-    int o;
-    if (pos <= nh)
-      o = pos;
-    else if (pos > n)
-      o = pos - nh;
-    else
-      return;
-    p[(long long)b * sb + (long long)o * sp + col] = v;
+  __device__ __forceinline__ void store(int b, int col, Pos pos, cx<T> v, cx<T>) const {
+    if (Kept::drop(pos)) return;
+    const Kept k(pos, n);
+    if (k.keep) *line_at(p + (long long)b * sb, sp, col, k.t, k.c) = v;
   }
 };
 
@@ -222,46 +272,29 @@ struct DstTruncOp {
   }
   // previous output value for the accumulating operators, loaded for every
   // element of the thread before any store (clamped index, no branch)
-  __device__ __forceinline__ cx<T> load_old(int b, int col, int pos) const {
-    if (op == OP_ASSIGN) return mk(T(0), T(0));
-    const int nh = n >> 1;
-    const bool drop = (pos > nh) & (pos <= n);
-    const int i = drop ? 0 : (pos <= nh ? pos : pos - nh);
+  __device__ __forceinline__ cx<T> load_old(int b, int col, Pos pos) const {
+    if (op == OP_ASSIGN || Kept::drop(pos)) return mk(T(0), T(0));
+    const Kept k(pos, n);
     const int q = b / nb;
-    return array(q)[(long long)i * sp + (long long)(b - q * nb) * sb + col];
+    return *line_at(array(q) + (long long)(b - q * nb) * sb, sp, col, k.t, k.c);
   }
-  // output value at retained index i of line set b, column col
-  __device__ __forceinline__ cx<T> value(int b, int col, int i, cx<T> v, cx<T> prev) const {
-    const int nh = n >> 1;
-    const bool nyq = (i == nh) | (b == nh) | (col == nh);
-    cx<T> val = nyq ? mk(T(0), T(0)) : v * scale;
-    cx<T> o;
-    if (op == OP_ASSIGN)
-      o = val;
-    else if (op == OP_ADD)
-      o = prev + val;
-    else if (op == OP_SUB)
-      o = prev - val;
-    else
-      o = prev + val * opfac;
+  // The value is formed without a branch and only its store is predicated: what
+  // does not depend on the element is then computed once for each thread.
+  __device__ __forceinline__ void store(int b, int col, Pos pos, cx<T> v, cx<T> prev) const {
+    if (Kept::drop(pos)) return;
+    const Kept k(pos, n);
+    const int nh = n >> 1, q = b / nb, j = b - q * nb;
+    const bool nyq = k.nyq | (j == nh) | (col == nh);
+    const T w = op == OP_SUB ? T(-1) : (op == OP_MULADD ? opfac : T(1));
+    const cx<T> val = nyq ? mk(T(0), T(0)) : v * scale;
+    cx<T> o = prev + val * w;  // prev is zero for the assignment
     if (invlap) {
-      T kx = kval<T>(i, n, kfac, 0), ky = kval<T>(b, n, kfac, 0), kz = kval<T>(col, n, kfac, 0);
-      T k2 = kx * kx + ky * ky + kz * kz;
-      o = (i == 0 && b == 0 && col == 0) ? mk(T(0), T(0)) : mk(-o.x / k2, -o.y / k2);
+      const T ky = kval<T>(j, n, kfac, 0), kz = kval<T>(col, n, kfac, 0), kx = T(k.t + k.k0) * kfac;
+      const T k2 = kx * kx + ky * ky + kz * kz;
+      const bool dc = (k.t + k.c == 0) & (j == 0) & (col == 0);
+      o = dc ? mk(T(0), T(0)) : mk(-o.x / k2, -o.y / k2);
     }
-    return o;
-  }
-  __device__ __forceinline__ void store(int b, int col, int pos, cx<T> v, cx<T> prev) const {
-    const int nh = n >> 1;
-    int i;
-    if (pos <= nh)
-      i = pos;
-    else if (pos > n)
-      i = pos - nh;
-    else
-      return;
-    const int q = b / nb, j = b - q * nb;
-    array(q)[(long long)i * sp + (long long)j * sb + col] = value(j, col, i, v, prev);
+    if (k.keep) *line_at(array(q) + (long long)j * sb, sp, col, k.t, k.c) = o;
   }
 };
 
@@ -281,9 +314,9 @@ struct DstPhi1 {
   const double* amp;
   NoiseNorm nn;
   __device__ __forceinline__ cx<T> load_old(int, int, int) const { return mk(T(0), T(0)); }
-  __device__ __forceinline__ void store(int, int col, int pos, cx<T> v, cx<T>) const {
+  __device__ __forceinline__ void store(int, int col, Pos pos, cx<T> v, cx<T>) const {
     const int j = col / H;
-    phi[(long long)pos * sp + col] = phi1_value(v * scale, pos, j, col - j * H, n, kfac, amp, nn);
+    *line_at(phi, sp, col, pos.t, pos.c) = phi1_value(v * scale, pos, j, col - j * H, n, kfac, amp, nn);
   }
 };
 
@@ -301,8 +334,8 @@ __device__ __forceinline__ void xcd_tile(int& tile, int& b) {
   const long long per = total / NX, rem = total % NX;
   const long long x = id % NX, local = id / NX;
   const long long w = (x < rem) ? x * (per + 1) + local : rem * (per + 1) + (x - rem) * per + local;
-  tile = (int)(w % ntiles);
-  b = (int)(w / ntiles);
+  tile = __builtin_amdgcn_readfirstlane((int)(w % ntiles));
+  b = __builtin_amdgcn_readfirstlane((int)(w / ntiles));
 }
 
 // C adjacent columns per workgroup (the tile width chosen by the autotuner)
@@ -310,7 +343,7 @@ template <typename T, int L, bool INV, class Src, class Dst, int C, int V = 0>
 __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
     k_col(Src src, Dst dst, const cx<T>* __restrict__ tw, int ncols) {
   constexpr int EPT = PlanInfo<L, V>::EPT, TPS = PlanInfo<L, V>::TPS;
-  extern __shared__ __align__(16) unsigned char col_lds_raw[];  // TwLds<T, L, C>::bytes
+  extern __shared__ __align__(16) unsigned char col_lds_raw[];  // TwLds<T, L, C, V>::bytes
   cx<T>* const lds = reinterpret_cast<cx<T>*>(col_lds_raw);
   cx<T>* const twl = lds + L * C;
   const int c = threadIdx.x % C, t = threadIdx.x / C;
@@ -322,15 +355,15 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
   const int colc = act ? col : ncols - 1;
   cx<T> v[EPT];
 #pragma unroll
-  for (int e = 0; e < EPT; ++e) v[e] = src.load(b, colc, t + TPS * e);
+  for (int e = 0; e < EPT; ++e) v[e] = src.load(b, colc, Pos(t, TPS * e, TPS, L));
   const ColTw<T, L, C, V> ft(tw, twl);  // after the loads: their latency overlaps the table copy
   ft.template exec<INV>(v, lds + c, C, t);
   cx<T> old[EPT];
 #pragma unroll
-  for (int e = 0; e < EPT; ++e) old[e] = dst.load_old(b, colc, t + TPS * e);
+  for (int e = 0; e < EPT; ++e) old[e] = dst.load_old(b, colc, Pos(t, TPS * e, TPS, L));
   if (act) {
 #pragma unroll
-    for (int e = 0; e < EPT; ++e) dst.store(b, col, t + TPS * e, v[e], old[e]);
+    for (int e = 0; e < EPT; ++e) dst.store(b, col, Pos(t, TPS * e, TPS, L), v[e], old[e]);
   }
 }
 
@@ -357,7 +390,7 @@ template <typename T, int L, bool INV, class Src, class Dst, int C, int V = 0>
 __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
     k_col_pipe(Src src, Dst dst, const cx<T>* __restrict__ tw, int ncols, int ntiles, long long nitems) {
   constexpr int EPT = PlanInfo<L, V>::EPT, TPS = PlanInfo<L, V>::TPS;
-  extern __shared__ __align__(16) unsigned char col_lds_raw[];  // TwLds<T, L, C>::bytes
+  extern __shared__ __align__(16) unsigned char col_lds_raw[];  // TwLds<T, L, C, V>::bytes
   cx<T>* const lds = reinterpret_cast<cx<T>*>(col_lds_raw);
   cx<T>* const twl = lds + L * C;
   const int c = threadIdx.x % C, t = threadIdx.x / C;
@@ -366,10 +399,11 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
   if (!pipe_range(nitems, w, hi, step)) return;
   cx<T> nx[EPT];
   auto fetch = [&](long long item, int tq, cx<T>(&v)[EPT]) {
-    const int b = (int)(item / ntiles), col = (int)(item % ntiles) * C + c;
+    const int b = __builtin_amdgcn_readfirstlane((int)(item / ntiles)),
+              col = __builtin_amdgcn_readfirstlane((int)(item % ntiles)) * C + c;
     const int colc = col < ncols ? col : ncols - 1;
 #pragma unroll
-    for (int e = 0; e < EPT; ++e) v[e] = src.load(b, colc, tq + TPS * e);
+    for (int e = 0; e < EPT; ++e) v[e] = src.load(b, colc, Pos(tq, TPS * e, TPS, L));
   };
   fetch(w, t, nx);
   const ColTw<T, L, C, V> ft(tw, twl);
@@ -385,14 +419,15 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
     // every stage exchange of the previous item ended with a barrier after
     // its last LDS read, so the first exchange of this one may write
     ft.template exec<INV>(v, lds + c, C, t);
-    const int b = (int)(w / ntiles), col = (int)(w % ntiles) * C + c;
+    const int b = __builtin_amdgcn_readfirstlane((int)(w / ntiles)),
+              col = __builtin_amdgcn_readfirstlane((int)(w % ntiles)) * C + c;
     const int colc = col < ncols ? col : ncols - 1;
     cx<T> old[EPT];
 #pragma unroll
-    for (int e = 0; e < EPT; ++e) old[e] = dst.load_old(b, colc, tq + TPS * e);
+    for (int e = 0; e < EPT; ++e) old[e] = dst.load_old(b, colc, Pos(tq, TPS * e, TPS, L));
     if (col < ncols) {
 #pragma unroll
-      for (int e = 0; e < EPT; ++e) dst.store(b, col, tq + TPS * e, v[e], old[e]);
+      for (int e = 0; e < EPT; ++e) dst.store(b, col, Pos(tq, TPS * e, TPS, L), v[e], old[e]);
     }
   }
 }
@@ -417,12 +452,12 @@ struct MultiPow {
   cx<T>* out[3];
   int pw[3];
   int no;
-  __device__ __forceinline__ cx<T> load(int o, int b, int col, int pos) const {
+  __device__ __forceinline__ cx<T> load(int o, int b, int col, Pos pos) const {
     SrcPadPow<T> s = src;
     s.pw = o == 0 ? pw[0] : (o == 1 ? pw[1] : pw[2]);
     return s.load(b, col, pos);
   }
-  __device__ __forceinline__ void store(int o, int b, int col, int pos, cx<T> v) const {
+  __device__ __forceinline__ void store(int o, int b, int col, Pos pos, cx<T> v) const {
     DstPlain<T> d = dst;
     d.p = o == 0 ? out[0] : (o == 1 ? out[1] : out[2]);
     d.store(b, col, pos, v, v);
@@ -433,7 +468,7 @@ template <typename T, int L, bool INV, int C, int V, class M>
 __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
     k_col_multi(M a, const cx<T>* __restrict__ tw, int ncols) {
   constexpr int EPT = PlanInfo<L, V>::EPT, TPS = PlanInfo<L, V>::TPS;
-  extern __shared__ __align__(16) unsigned char col_lds_raw[];  // TwLds<T, L, C>::bytes
+  extern __shared__ __align__(16) unsigned char col_lds_raw[];  // TwLds<T, L, C, V>::bytes
   cx<T>* const lds = reinterpret_cast<cx<T>*>(col_lds_raw);
   cx<T>* const twl = lds + L * C;
   const int c = threadIdx.x % C, t = threadIdx.x / C;
@@ -453,13 +488,13 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
     asm volatile("" : "+v"(tq), "+v"(cq), "+v"(colq));
     cx<T> v[EPT];
 #pragma unroll
-    for (int e = 0; e < EPT; ++e) v[e] = a.load(o, b, cq, tq + TPS * e);
+    for (int e = 0; e < EPT; ++e) v[e] = a.load(o, b, cq, Pos(tq, TPS * e, TPS, L));
     // the previous output's last exchange ended with a barrier after its
     // last LDS read, so this transform's first exchange may write
     ft.template exec<INV>(v, lds + c, C, t);
     if (act) {
 #pragma unroll
-      for (int e = 0; e < EPT; ++e) a.store(o, b, colq, tq + TPS * e, v[e]);
+      for (int e = 0; e < EPT; ++e) a.store(o, b, colq, Pos(tq, TPS * e, TPS, L), v[e]);
     }
   }
 }
@@ -470,14 +505,14 @@ template <typename T, class M>
 struct MultiSrc {
   M m;
   int o;
-  __device__ __forceinline__ cx<T> load(int b, int col, int pos) const { return m.load(o, b, col, pos); }
+  __device__ __forceinline__ cx<T> load(int b, int col, Pos pos) const { return m.load(o, b, col, pos); }
 };
 template <typename T, class M>
 struct MultiDst {
   M m;
   int o;
   __device__ __forceinline__ cx<T> load_old(int, int, int) const { return mk(T(0), T(0)); }
-  __device__ __forceinline__ void store(int b, int col, int pos, cx<T> v, cx<T>) const { m.store(o, b, col, pos, v); }
+  __device__ __forceinline__ void store(int b, int col, Pos pos, cx<T> v, cx<T>) const { m.store(o, b, col, pos, v); }
 };
 
 // Projection of a padded line onto the modes of the n-grid: forward
@@ -509,11 +544,20 @@ struct TurnArgs {
   }
 };
 
+// whether position t + c (c .. c + W - 1 the element's range) of a padded line of
+// L = 3n/2 positions is dropped or the Nyquist one: n/2 .. n
+__device__ __forceinline__ bool turn_zero(int t, int c, int W, int L) {
+  const int nh = L / 3, n = 2 * (L / 3);
+  if (c + W - 1 < nh || c > n) return false;
+  if (c >= nh && c + W - 1 <= n) return true;
+  return (t + c >= nh) & (t + c <= n);
+}
+
 template <typename T, int L, int C, int V = 0>
 __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
     k_col_turn(TurnArgs<T> a, const cx<T>* __restrict__ tw, int ncols) {
   constexpr int EPT = PlanInfo<L, V>::EPT, TPS = PlanInfo<L, V>::TPS;
-  extern __shared__ __align__(16) unsigned char col_lds_raw[];  // TwLds<T, L, C>::bytes
+  extern __shared__ __align__(16) unsigned char col_lds_raw[];  // TwLds<T, L, C, V>::bytes
   cx<T>* const lds = reinterpret_cast<cx<T>*>(col_lds_raw);
   cx<T>* const twl = lds + L * C;
   const int c = threadIdx.x % C, t = threadIdx.x / C;
@@ -526,15 +570,14 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
   const cx<T>* const from = a.from(b);
   cx<T> x[EPT];
 #pragma unroll
-  for (int e = 0; e < EPT; ++e) x[e] = from[(long long)(t + TPS * e) * a.sp + colc];
+  for (int e = 0; e < EPT; ++e) x[e] = *line_at(from, a.sp, colc, t, TPS * e);
   const ColTw<T, L, C, V> ft(tw, twl);
   ft.template exec<false>(x, lds + c, C, t);
   const bool nyqc = colc == nh;
 #pragma unroll
   for (int e = 0; e < EPT; ++e) {
-    const int pos = t + TPS * e;
-    // dropped positions and the Nyquist mode (index n/2 is position n/2)
-    const bool zero = ((pos > nh) & (pos <= a.n)) | (pos == nh) | nyqc;
+    // dropped positions and the Nyquist mode (index n/2 is position n/2 = L/3)
+    const bool zero = turn_zero(t, TPS * e, TPS, L) | nyqc;
     const cx<T> o = x[e] * a.fscale;  // the n-grid value
     x[e] = zero ? mk(T(0), T(0)) : o * a.iscale;
   }
@@ -543,7 +586,7 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
   if (act) {
     cx<T>* const to = a.to(b);
 #pragma unroll
-    for (int e = 0; e < EPT; ++e) to[(long long)(t + TPS * e) * a.osp + col] = x[e];
+    for (int e = 0; e < EPT; ++e) *line_at(to, a.osp, col, t, TPS * e) = x[e];
   }
 }
 
@@ -552,7 +595,7 @@ template <typename T, int L, int C, int V = 0>
 __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
     k_col_turn_pipe(TurnArgs<T> a, const cx<T>* __restrict__ tw, int ncols, int ntiles, long long nitems) {
   constexpr int EPT = PlanInfo<L, V>::EPT, TPS = PlanInfo<L, V>::TPS;
-  extern __shared__ __align__(16) unsigned char col_lds_raw[];  // TwLds<T, L, C>::bytes
+  extern __shared__ __align__(16) unsigned char col_lds_raw[];  // TwLds<T, L, C, V>::bytes
   cx<T>* const lds = reinterpret_cast<cx<T>*>(col_lds_raw);
   cx<T>* const twl = lds + L * C;
   const int c = threadIdx.x % C, t = threadIdx.x / C;
@@ -562,11 +605,12 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
   if (!pipe_range(nitems, w, hi, step)) return;
   cx<T> nx[EPT];
   auto fetch = [&](long long item, int tq, cx<T>(&v)[EPT]) {
-    const int b = (int)(item / ntiles), col = (int)(item % ntiles) * C + c;
+    const int b = __builtin_amdgcn_readfirstlane((int)(item / ntiles)),
+              col = __builtin_amdgcn_readfirstlane((int)(item % ntiles)) * C + c;
     const int colc = col < ncols ? col : ncols - 1;
     const cx<T>* const from = a.from(b);
 #pragma unroll
-    for (int e = 0; e < EPT; ++e) v[e] = from[(long long)(tq + TPS * e) * a.sp + colc];
+    for (int e = 0; e < EPT; ++e) v[e] = *line_at(from, a.sp, colc, tq, TPS * e);
   };
   fetch(w, t, nx);
   const ColTw<T, L, C, V> ft(tw, twl);
@@ -577,14 +621,14 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
 #pragma unroll
     for (int e = 0; e < EPT; ++e) x[e] = nx[e];
     if (w + step < hi) fetch(w + step, tq, nx);
-    const int b = (int)(w / ntiles), col = (int)(w % ntiles) * C + c;
+    const int b = __builtin_amdgcn_readfirstlane((int)(w / ntiles)),
+              col = __builtin_amdgcn_readfirstlane((int)(w % ntiles)) * C + c;
     const int colc = col < ncols ? col : ncols - 1;
     ft.template exec<false>(x, lds + c, C, t);
     const bool nyqc = colc == nh;
 #pragma unroll
     for (int e = 0; e < EPT; ++e) {
-      const int pos = tq + TPS * e;
-      const bool zero = ((pos > nh) & (pos <= a.n)) | (pos == nh) | nyqc;
+      const bool zero = turn_zero(tq, TPS * e, TPS, L) | nyqc;
       const cx<T> o = x[e] * a.fscale;
       x[e] = zero ? mk(T(0), T(0)) : o * a.iscale;
     }
@@ -593,7 +637,7 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
     if (col < ncols) {
       cx<T>* const to = a.to(b);
 #pragma unroll
-      for (int e = 0; e < EPT; ++e) to[(long long)(tq + TPS * e) * a.osp + col] = x[e];
+      for (int e = 0; e < EPT; ++e) *line_at(to, a.osp, col, tq, TPS * e) = x[e];
     }
   }
 }
@@ -638,7 +682,7 @@ void launch_col_LC(Ctx& c, Src s, Dst d, int ncols, int nbatch, const char* name
   const dim3 block(C * PlanInfo<L, V>::TPS);
   const int ntiles = (ncols + C - 1) / C;
   LaunchScope ls(c, name, bytes);
-  constexpr size_t dyn = TwLds<T, L, C>::bytes;
+  constexpr size_t dyn = TwLds<T, L, C, V>::bytes;
   if constexpr (PIPE) {
     const long long nitems = (long long)ntiles * nbatch;
     auto k = k_col_pipe<T, L, INV, Src, Dst, C, V>;
@@ -828,7 +872,7 @@ void launch_turn_LC(Ctx& c, const TurnArgs<T>& a, int ncols, int nbatch, const c
   const dim3 block(C * PlanInfo<L, V>::TPS);
   const int ntiles = (ncols + C - 1) / C;
   LaunchScope ls(c, name, bytes);
-  constexpr size_t dyn = TwLds<T, L, C>::bytes;
+  constexpr size_t dyn = TwLds<T, L, C, V>::bytes;
   if constexpr (PIPE) {
     const long long nitems = (long long)ntiles * nbatch;
     auto k = k_col_turn_pipe<T, L, C, V>;
@@ -903,7 +947,7 @@ void launch_multi_LC(Ctx& c, const M& a, int ncols, int nbatch, const char* name
   const dim3 block(C * PlanInfo<L, V>::TPS);
   const int ntiles = (ncols + C - 1) / C;
   LaunchScope ls(c, name, bytes);
-  constexpr size_t dyn = TwLds<T, L, C>::bytes;
+  constexpr size_t dyn = TwLds<T, L, C, V>::bytes;
   auto k = k_col_multi<T, L, INV, C, V, M>;
   col_lds_prep(c, k, dyn);
   hipLaunchKernelGGL(k, dim3(ntiles, nbatch), block, dyn, c.stream, a, c.twiddles<T>(L), ncols);

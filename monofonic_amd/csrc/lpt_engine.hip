@@ -572,7 +572,8 @@ struct Engine {
   // launch each: all of them where they fit the 256 MiB memory-side cache with
   // room to spare (a chain's next pass then still finds them there, and a small
   // grid's launches, whose 4 to 15 us hardly depend on the work, are fewer), one at
-  // a time where a single array does not (LPT_FIGURES).
+  // a time where a single array does not (96^3 FP64: the eight projections 117 -> 75 us,
+  // the ten forward passes 122 -> 98 us; 512^3: unchanged).
   static int together(int cnt, double bytes) {
     const int fit = (int)(160.0 * (1 << 20) / bytes);
     const int groups = fit < 1 ? cnt : (cnt + fit - 1) / fit;

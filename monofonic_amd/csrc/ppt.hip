@@ -165,7 +165,7 @@ template <typename T, int L, int C, class Src, class Dst, class Mul>
 __global__ void __launch_bounds__((C * PlanInfo<L, 0>::TPS))
     k_col_fwd_mul_inv(Src src, Dst dst, Mul mul, const cx<T>* __restrict__ tw, int ncols) {
   constexpr int EPT = PlanInfo<L, 0>::EPT, TPS = PlanInfo<L, 0>::TPS;
-  extern __shared__ __align__(16) unsigned char col_lds_raw[];  // TwLds<T, L, C>::bytes
+  extern __shared__ __align__(16) unsigned char col_lds_raw[];  // TwLds<T, L, C, 0>::bytes
   cx<T>* const lds = reinterpret_cast<cx<T>*>(col_lds_raw);
   cx<T>* const twl = lds + L * C;
   const int c = threadIdx.x % C, t = threadIdx.x / C;
@@ -176,7 +176,7 @@ __global__ void __launch_bounds__((C * PlanInfo<L, 0>::TPS))
   const int colc = act ? col : ncols - 1;
   cx<T> v[EPT];
 #pragma unroll
-  for (int e = 0; e < EPT; ++e) v[e] = src.load(b, colc, t + TPS * e);
+  for (int e = 0; e < EPT; ++e) v[e] = src.load(b, colc, Pos(t, TPS * e, TPS, L));
   const ColTw<T, L, C, 0> ft(tw, twl);
   ft.template exec<false>(v, lds + c, C, t);
 #pragma unroll
@@ -184,7 +184,7 @@ __global__ void __launch_bounds__((C * PlanInfo<L, 0>::TPS))
   ft.template exec<true>(v, lds + c, C, t);
   if (act) {
 #pragma unroll
-    for (int e = 0; e < EPT; ++e) dst.store(b, col, t + TPS * e, v[e], mk(T(0), T(0)));
+    for (int e = 0; e < EPT; ++e) dst.store(b, col, Pos(t, TPS * e, TPS, L), v[e], mk(T(0), T(0)));
   }
 }
 
@@ -192,7 +192,7 @@ template <typename T, int L, class Src, class Dst, class Mul>
 void launch_fmi_L(Ctx& c, Src s, Dst d, Mul m, int ncols, int nbatch, const char* name, double bytes) {
   constexpr int C = ColCfg<T, L>::C;
   const dim3 block(C * PlanInfo<L, 0>::TPS);
-  constexpr size_t dyn = TwLds<T, L, C>::bytes;
+  constexpr size_t dyn = TwLds<T, L, C, 0>::bytes;
   auto k = k_col_fwd_mul_inv<T, L, C, Src, Dst, Mul>;
   col_lds_prep(c, k, dyn);
   LaunchScope ls(c, name, bytes);
