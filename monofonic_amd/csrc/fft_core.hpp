@@ -373,31 +373,86 @@ constexpr int tw_count() {
   return most + 1;
 }
 
+// Exchange of a stage's outputs through an area of L real values a line: the real
+// parts, then the imaginary parts.  Half the LDS of fft_stage's exchange for
+// twice its barriers.
+template <typename T, int L, int EPT, int R, int NS>
+__device__ __forceinline__ void exchange_parts(cx<T> (&v)[EPT], T* lds, int ls, int t) {
+  constexpr int TPS = L / EPT, NB = EPT / R;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int m = 0; m < NB; ++m) {
+      const int j = t + TPS * m, base = (j / NS) * NS * R + j % NS;
+#pragma unroll
+      for (int q = 0; q < R; ++q) lds[(base + q * NS) * ls] = h ? v[m + q * NB].y : v[m + q * NB].x;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < EPT; ++e) {
+      const T x = lds[(t + TPS * e) * ls];
+      if (h)
+        v[e].y = x;
+      else
+        v[e].x = x;
+    }
+    __syncthreads();
+  }
+}
+
+template <typename T, int L, bool INV, int S, int V, int EPT, class TP>
+__device__ __forceinline__ void stage_loop_parts(cx<T> (&v)[EPT], T* lds, int ls, int t, TP tw) {
+  using P = Plan<L, V>;
+  if constexpr (S < P::NR) {
+    constexpr int R = P::R[S], NS = StageNS<L, S, V>::value;
+    cx<T> w[EPT];
+    stage_twiddles<T, L, S, V>(w, tw, t);
+    fft_stage<T, L, EPT, R, NS, INV, true>(v, nullptr, 0, t, w);  // outputs stay in registers
+    if constexpr (S + 1 < P::NR) exchange_parts<T, L, EPT, R, NS>(v, lds, ls, t);
+    stage_loop_parts<T, L, INV, S + 1, V>(v, lds, ls, t, tw);
+  }
+}
+
 // LDS layout of a column workgroup of C lines of length L (plan V), all in
-// dynamic LDS: the exchange area (L*C values) followed by the twiddles the plan
-// reads, at most 3/4 of the table after a first radix of 12.  768-line FP32 tiles of
-// 8 columns then take 52.5 KiB, three workgroups on a compute unit's 160 KiB; with
-// the whole table two fit, and with half of it (w^(i + L/2) = -w^i by selects) a
-// tenth of the kernel's instructions were those selects.
+// dynamic LDS: the exchange area followed by the twiddles the plan reads, at most
+// 3/4 of the table after a first radix of 12.  768-line FP32 tiles of 8 columns
+// then take 52.5 KiB, three workgroups on a compute unit's 160 KiB; with the whole
+// table two fit, and with half of it (w^(i + L/2) = -w^i by selects) a tenth of the
+// kernel's instructions were those selects.
+// The area holds L*C complex values where these fit 64 KiB, else (the wide tiles)
+// L*C real ones (exchange_parts): 16 FP32 columns of 768 in 52.5 KiB, two
+// workgroups of 1024 threads on a compute unit where the complex area allows one.
+// The y stage of the Hessian rows at 768 then takes 0.342 ms for 128 planes (FP32,
+// streaming stores, 4.7 TB/s) against 0.480 with the complex area and 0.473 with 8
+// columns; FP64 (8 columns) 0.322 against 0.436 and 0.476.
 template <typename T, int L, int C, int V>
 struct TwLds {
   static constexpr int entries = tw_count<L, V>();
-  static constexpr size_t bytes = (size_t)((long long)L * C + entries) * sizeof(cx<T>);
+  static constexpr bool parts = (long long)L * C * sizeof(cx<T>) > 65536;
+  static constexpr size_t area = (size_t)L * C * (parts ? sizeof(T) : sizeof(cx<T>));
+  static constexpr size_t bytes = area + (size_t)entries * sizeof(cx<T>);
 };
 
-// Copies the twiddles (TwLds::entries values) into LDS at lt and runs the
-// transforms through them.  Construct once per workgroup, before any transform;
-// the constructor ends with a barrier.
+// Copies the twiddles (TwLds::entries values) into LDS behind the exchange area
+// at raw and runs the transforms of the workgroup's C lines through both: exec()
+// for the thread's elements (position t) of line c.  Construct once per workgroup,
+// before any transform; the constructor ends with a barrier.
 template <typename T, int L, int C, int V>
 struct ColTw {
+  using Lds = TwLds<T, L, C, V>;
+  unsigned char* raw;
   cx<T>* s;
-  __device__ __forceinline__ ColTw(const cx<T>* tw, cx<T>* lt) : s(lt) {
-    for (int i = threadIdx.x; i < TwLds<T, L, C, V>::entries; i += blockDim.x) s[i] = tw[i];
+  __device__ __forceinline__ ColTw(const cx<T>* tw, unsigned char* raw_)
+      : raw(raw_), s(reinterpret_cast<cx<T>*>(raw_ + Lds::area)) {
+    for (int i = threadIdx.x; i < Lds::entries; i += blockDim.x) s[i] = tw[i];
     __syncthreads();
   }
   template <bool INV, int EPT>
-  __device__ __forceinline__ void exec(cx<T> (&v)[EPT], cx<T>* lds, int ls, int t) const {
-    fft_exec_lt<T, L, INV, V>(v, lds, ls, t, s);
+  __device__ __forceinline__ void exec(cx<T> (&v)[EPT], int c, int t) const {
+    if constexpr (Lds::parts)
+      stage_loop_parts<T, L, INV, 0, V>(v, reinterpret_cast<T*>(raw) + c, C, t, lds_table(s));
+    else
+      fft_exec_lt<T, L, INV, V>(v, reinterpret_cast<cx<T>*>(raw) + c, C, t, s);
   }
 };
 

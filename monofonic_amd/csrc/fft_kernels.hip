@@ -210,13 +210,16 @@ void conv2(Ctx& c, const cx<T>* fa, const MultSpec& ma, const cx<T>* fb, const M
 // more elements per thread.  Which is faster depends on the length and
 // precision, so the (up to) twelve combinations are timed on a block of the library's own shape -- L/2+1
 // adjacent columns, up to 256 batches -- in both directions, five launches
-// each after two warm-ups, and the fastest is kept.
+// each after two warm-ups, and the fastest is kept.  Lengths 3n/2 are timed on
+// the work grids' n/2 + 1 columns at their padded pitch, the only one that all
+// columns of a tile can be streamed to.
 template <typename T>
 void autotune_columns(Ctx& c, int L) {
   const int cm = col_tile_max<T>(L);
-  const int ncols = L / 2 + 1;
+  const int ncols = L % 3 == 0 ? L / 3 + 1 : L / 2 + 1;
+  const int pitch = L % 3 == 0 ? conv_pitch(2 * L / 3) : ncols;
   const int nb = L < 256 ? L : 256;
-  const long long cnt = (long long)nb * L * ncols;
+  const long long cnt = (long long)nb * L * pitch;
   cx<T>* buf = reinterpret_cast<cx<T>*>(c.alloc(sizeof(cx<T>) * cnt));
   hipEvent_t e0 = nullptr, e1 = nullptr;
   const bool prof = c.profile;
@@ -259,20 +262,35 @@ void autotune_columns(Ctx& c, int L) {
       // class 0: lines of L elements a row of columns apart ([batch][line][col]);
       // class 1: a plane apart ([line][batch][col]); only where the plane is
       // large enough to be class 1 at all
-      const long long sb = cls ? ncols : (long long)L * ncols, sp = cls ? (long long)nb * ncols : ncols;
+      const long long sb = cls ? pitch : (long long)L * pitch, sp = cls ? (long long)nb * pitch : pitch;
       if (stride_class(sp, (int)sizeof(cx<T>)) != cls) continue;
-      for (int inv = 0; inv < 2; ++inv)
+      const bool padded = L % 3 == 0 && (L / 3) % 2 == 0;
+      const int nn = 2 * L / 3;
+      for (int inv = 0; inv < 2; ++inv) {
+        // at a padded length the row-strided inverse pass is the y stage of the
+        // Hessian rows: six outputs of three sources, as many planes as the block
+        // holds.  An in-place pass prefers other variants: 384-line FP64 1.94 ms of
+        // its choice against 1.00, 768-line FP32 4.72 against 4.15 (two fields)
+        const int planes = (int)((long long)nb * L / (3ll * nn + 6ll * L));
+        if (padded && inv && cls == 0 && planes > 0) {
+          const long long xs = (long long)planes * nn * pitch, ys = (long long)planes * L * pitch;
+          cx<T>* const y = buf + 3 * xs;
+          const SrcHessY<T> hs{{buf, buf + xs, buf + 2 * xs}, (long long)nn * pitch, pitch, nn, T(1)};
+          const DstHessY<T> hd{{y, y + ys, y + 2 * ys, y + 3 * ys, y + 4 * ys, y + 5 * ys}, sb, sp};
+          tune(inv, cls, true, [&] { launch_hess_y<T>(c, L, hs, hd, ncols, planes, "tune", 0); });
+          continue;
+        }
         tune(inv, cls, true, [&] {
           if (inv)
             launch_col<T, true>(c, L, SrcPlain<T>{buf, sb, sp}, DstPlain<T>{buf, sb, sp, T(1)}, ncols, nb, "tune", 0);
           else
             launch_col<T, false>(c, L, SrcPlain<T>{buf, sb, sp}, DstPlain<T>{buf, sb, sp, T(1)}, ncols, nb, "tune", 0);
         });
+      }
       // the projection (turn) passes of the padded lengths M = 3n/2, in place
       // as in the LPT engine: two transforms per line and more registers than
       // a plain pass, so they are tuned on their own
-      if (L % 3 == 0 && (L / 3) % 2 == 0) {
-        const int nn = 2 * L / 3;
+      if (padded) {
         const TurnArgs<T> ta{buf, sb, sp, nn, T(1), T(1), buf, sb, sp, nb, 0, 0};
         tune(COL_TURN, cls, true, [&] { launch_turn<T>(c, L, ta, ncols, nb, "tune", 0); });
         // the truncating forward pass with an output operator (the last x

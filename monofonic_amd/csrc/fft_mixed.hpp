@@ -334,6 +334,13 @@ __global__ void __launch_bounds__(1024)
 #pragma unroll
     for (int q = 0; q < R; ++q) old[q] = dst.load_old(b, colc, k + q * K);
     if (act) {
+      if constexpr (Streams<Dst>::value) {
+        if (dst.nt) {
+#pragma unroll
+          for (int q = 0; q < R; ++q) dst.template store<true>(b, col, k + q * K, a[q], old[q]);
+          return;
+        }
+      }
 #pragma unroll
       for (int q = 0; q < R; ++q) dst.store(b, col, k + q * K, a[q], old[q]);
     }
@@ -359,7 +366,7 @@ __device__ __forceinline__ void mix_turn_run(cx<T>* x, int ls, const MixPlan& p,
       const int k = k0 + q * nb;
       const bool zero = ((k > nh) & (k <= n)) | (k == nh) | nyqc;
       const cx<T> o = a[q] * fscale;  // the n-grid value
-      a[q] = zero ? mk(T(0), T(0)) : o * iscale;
+      a[q] = or_zero(!zero, o * iscale);
     }
     BF<R, true, T>::run(a);
 #pragma unroll
@@ -419,8 +426,13 @@ __global__ void __launch_bounds__(1024)
   auto done = [&](cx<T>* v, int k, int K, auto r) {
     constexpr int R = decltype(r)::value;
     if (act) {
+      if (a.nt) {
 #pragma unroll
-      for (int q = 0; q < R; ++q) out[(long long)(k + q * K) * a.osp] = v[q];
+        for (int q = 0; q < R; ++q) put<true>(out + (long long)(k + q * K) * a.osp, v[q]);
+      } else {
+#pragma unroll
+        for (int q = 0; q < R; ++q) out[(long long)(k + q * K) * a.osp] = v[q];
+      }
     }
   };
   switch (p.R[0].d) {

@@ -9,7 +9,9 @@
 #include "row_fft.hpp"
 
 #include <cmath>
+#include <cstdint>
 #include <string>
+#include <type_traits>
 
 namespace mfx {
 
@@ -91,6 +93,44 @@ struct Pos {
   __device__ __forceinline__ operator int() const { return t + c; }
 };
 
+// Streaming (non-temporal) stores of a column pass: only where every line of a
+// tile of C columns is whole 128-byte cache lines (run C*sizeof(cx), base and
+// strides all multiples of 128 bytes, as in the padded work grids); a partial
+// line stored past the L2 costs a read and write of the whole line.  Plain passes
+// of 257 columns (FP32; GB/s without -> with): 768 lines, pitch 272, 16 columns:
+// out of place 4627 -> 5232 (y), 4154 -> 4669 (x), in place 4111 -> 4731, 3834 ->
+// 4343; 8 columns (64-byte runs) 4313 -> 4088; 512 lines, pitch 257: 4982 -> 2616.
+// FP64, 384 lines, 8 columns in place (y) 5201 -> 6678.
+inline bool streams(const void* p, int C, long long sb, long long sp, size_t size) {
+  return (C * size) % 128 == 0 && ((unsigned long long)sb * size) % 128 == 0 &&
+         ((unsigned long long)sp * size) % 128 == 0 && (reinterpret_cast<uintptr_t>(p) & 127) == 0;
+}
+
+template <bool NT, typename T>
+__device__ __forceinline__ void put(cx<T>* p, cx<T> v) {
+  if constexpr (NT) {
+    typedef T pair __attribute__((ext_vector_type(2)));
+    __builtin_nontemporal_store(pair{v.x, v.y}, reinterpret_cast<pair*>(p));
+  } else {
+    *p = v;
+  }
+}
+
+// Whether a destination has a streaming form: a flag nt, set by stream(C) at the
+// launch, and store<true>.
+template <class D, class = void>
+struct Streams {
+  static constexpr bool value = false;
+};
+template <class D>
+struct Streams<D, std::void_t<decltype(&D::stream)>> {
+  static constexpr bool value = true;
+};
+template <class D>
+void set_stream(D& d, int C) {
+  if constexpr (Streams<D>::value) d.stream(C);
+}
+
 // element t + c of a line: column col of line set base (uniform), line stride sp
 template <typename C>
 __device__ __forceinline__ C* line_at(C* base, long long sp, int col, int t, int c) {
@@ -136,6 +176,18 @@ struct Kept {
   }
 };
 
+// v or zero by selects on values: a conditional expression of complex type is
+// compiled to a branch around the load of v, and the loads of a thread are then
+// waited for one by one (the y stage at 576 lines, FP32: 3.7 instead of 2.8 ms)
+template <typename T>
+__device__ __forceinline__ T pick(bool c, T a, T b) {
+  return c ? a : b;
+}
+template <typename T>
+__device__ __forceinline__ cx<T> or_zero(bool keep, cx<T> v) {
+  return mk(pick(keep, v.x, T(0)), pick(keep, v.y, T(0)));
+}
+
 template <typename T>
 struct SrcPlain {
   const cx<T>* p;
@@ -163,9 +215,12 @@ struct DstPlain {
   cx<T>* p;
   long long sb, sp;
   T scale;
+  int nt = 0;
+  void stream(int C) { nt = streams(p, C, sb, sp, sizeof(cx<T>)); }
   __device__ __forceinline__ cx<T> load_old(int, int, int) const { return mk(T(0), T(0)); }
+  template <bool NT = false>
   __device__ __forceinline__ void store(int b, int col, Pos pos, cx<T> v, cx<T>) const {
-    *line_at(p + (long long)b * sb, sp, col, pos.t, pos.c) = v * scale;
+    put<NT>(line_at(p + (long long)b * sb, sp, col, pos.t, pos.c), v * scale);
   }
 };
 
@@ -186,8 +241,7 @@ struct SrcPad {
     const Kept k(pos, n);
     cx<T> v = *line_at(p + (long long)b * sb, sp, col, k.t, k.c);
     if (MULT) v = cmul(v, m.eval(k.t + k.c, b, col, n, kfac));
-    v = v * scale;
-    return k.keep ? v : mk(T(0), T(0));
+    return or_zero(k.keep, v * scale);
   }
 };
 
@@ -203,10 +257,10 @@ struct SrcPadPow {
     if (Kept::drop(pos)) return mk(T(0), T(0));
     const Kept k(pos, n);
     const cx<T> x = *line_at(p + (long long)b * sb, sp, col, k.t, k.c);
-    const T g = k.nyq ? T(0) : T(k.t + k.k0) * kfac;
-    const T f1 = pw == 0 ? scale : scale * g;
-    const T f = pw == 2 ? f1 * g : f1;
-    return k.keep ? x * f : mk(T(0), T(0));
+    const T g = pick(k.nyq, T(0), T(k.t + k.k0) * kfac);
+    const T f1 = pick(pw == 0, scale, scale * g);
+    const T f = pick(pw == 2, f1 * g, f1);
+    return or_zero(k.keep, x * f);
   }
 };
 
@@ -233,11 +287,17 @@ template <typename T>
 struct DstHessY {
   cx<T>* y[6];
   long long sb, sp;
+  int nt = 0;
+  void stream(int C) {
+    nt = 1;
+    for (cx<T>* q : y) nt &= streams(q, C, sb, sp, sizeof(cx<T>));
+  }
   __device__ __forceinline__ cx<T> load_old(int, int, int) const { return mk(T(0), T(0)); }
+  template <bool NT = false>
   __device__ __forceinline__ void store(int b, int col, Pos pos, cx<T> v, cx<T>) const {
     const int plane = b / 6, o = b - 6 * plane;
     cx<T>* p = o < 2 ? (o == 0 ? y[0] : y[1]) : (o < 4 ? (o == 2 ? y[2] : y[3]) : (o == 4 ? y[4] : y[5]));
-    *line_at(p + (long long)plane * sb, sp, col, pos.t, pos.c) = v;
+    put<NT>(line_at(p + (long long)plane * sb, sp, col, pos.t, pos.c), v);
   }
 };
 
@@ -247,11 +307,14 @@ struct DstTrunc {
   cx<T>* p;
   long long sb, sp;
   int n;
+  int nt = 0;
+  void stream(int C) { nt = streams(p, C, sb, sp, sizeof(cx<T>)); }
   __device__ __forceinline__ cx<T> load_old(int, int, int) const { return mk(T(0), T(0)); }
+  template <bool NT = false>
   __device__ __forceinline__ void store(int b, int col, Pos pos, cx<T> v, cx<T>) const {
     if (Kept::drop(pos)) return;
     const Kept k(pos, n);
-    if (k.keep) *line_at(p + (long long)b * sb, sp, col, k.t, k.c) = v;
+    if (k.keep) put<NT>(line_at(p + (long long)b * sb, sp, col, k.t, k.c), v);
   }
 };
 
@@ -286,13 +349,13 @@ struct DstTruncOp {
     const int nh = n >> 1, q = b / nb, j = b - q * nb;
     const bool nyq = k.nyq | (j == nh) | (col == nh);
     const T w = op == OP_SUB ? T(-1) : (op == OP_MULADD ? opfac : T(1));
-    const cx<T> val = nyq ? mk(T(0), T(0)) : v * scale;
+    const cx<T> val = or_zero(!nyq, v * scale);
     cx<T> o = prev + val * w;  // prev is zero for the assignment
     if (invlap) {
       const T ky = kval<T>(j, n, kfac, 0), kz = kval<T>(col, n, kfac, 0), kx = T(k.t + k.k0) * kfac;
       const T k2 = kx * kx + ky * ky + kz * kz;
       const bool dc = (k.t + k.c == 0) & (j == 0) & (col == 0);
-      o = dc ? mk(T(0), T(0)) : mk(-o.x / k2, -o.y / k2);
+      o = or_zero(!dc, mk(-o.x / k2, -o.y / k2));
     }
     if (k.keep) *line_at(array(q) + (long long)j * sb, sp, col, k.t, k.c) = o;
   }
@@ -338,14 +401,45 @@ __device__ __forceinline__ void xcd_tile(int& tile, int& b) {
   b = __builtin_amdgcn_readfirstlane((int)(w / ntiles));
 }
 
+// waves per SIMD that a column kernel is compiled for: two workgroups of 1024
+// threads where their LDS allows it (the wide FP32 tiles, at most 64 VGPRs), else
+// what one workgroup needs.  The accumulating output operator takes 70 VGPRs and
+// would spill.
+template <typename T, int L, int C, int V, bool TWO = true>
+constexpr int col_waves() {
+  constexpr int threads = C * PlanInfo<L, V>::TPS;
+  return TWO && threads == 1024 && sizeof(T) == 4 && 2 * TwLds<T, L, C, V>::bytes <= (size_t)CU_LDS ? 8 : (threads + 255) / 256;
+}
+
+// a thread's elements of one line to a destination
+template <int TPS, int L, bool NT, typename T, int EPT, class Dst>
+__device__ __forceinline__ void store_elements(const Dst& dst, int b, int col, int t, const cx<T> (&v)[EPT],
+                                               const cx<T> (&old)[EPT]) {
+#pragma unroll
+  for (int e = 0; e < EPT; ++e)
+    if constexpr (NT)
+      dst.template store<true>(b, col, Pos(t, TPS * e, TPS, L), v[e], old[e]);
+    else
+      dst.store(b, col, Pos(t, TPS * e, TPS, L), v[e], old[e]);
+}
+template <int TPS, int L, typename T, int EPT, class Dst>
+__device__ __forceinline__ void store_line(const Dst& dst, int b, int col, int t, const cx<T> (&v)[EPT],
+                                           const cx<T> (&old)[EPT]) {
+  if constexpr (Streams<Dst>::value) {
+    if (dst.nt) {
+      store_elements<TPS, L, true>(dst, b, col, t, v, old);
+      return;
+    }
+  }
+  store_elements<TPS, L, false>(dst, b, col, t, v, old);
+}
+
 // C adjacent columns per workgroup (the tile width chosen by the autotuner)
 template <typename T, int L, bool INV, class Src, class Dst, int C, int V = 0>
-__global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
+__global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS), (col_waves<T, L, C, V, Streams<Dst>::value>()))
     k_col(Src src, Dst dst, const cx<T>* __restrict__ tw, int ncols) {
   constexpr int EPT = PlanInfo<L, V>::EPT, TPS = PlanInfo<L, V>::TPS;
   extern __shared__ __align__(16) unsigned char col_lds_raw[];  // TwLds<T, L, C, V>::bytes
-  cx<T>* const lds = reinterpret_cast<cx<T>*>(col_lds_raw);
-  cx<T>* const twl = lds + L * C;
   const int c = threadIdx.x % C, t = threadIdx.x / C;
   int tile, b;
   xcd_tile(tile, b);
@@ -356,15 +450,14 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
   cx<T> v[EPT];
 #pragma unroll
   for (int e = 0; e < EPT; ++e) v[e] = src.load(b, colc, Pos(t, TPS * e, TPS, L));
-  const ColTw<T, L, C, V> ft(tw, twl);  // after the loads: their latency overlaps the table copy
-  ft.template exec<INV>(v, lds + c, C, t);
+  const ColTw<T, L, C, V> ft(tw, col_lds_raw);  // after the loads: their latency overlaps the table copy
+  ft.template exec<INV>(v, c, t);
+  int ts = t;  // the stores' addresses are formed here, not before the transform
+  asm volatile("" : "+v"(ts));
   cx<T> old[EPT];
 #pragma unroll
-  for (int e = 0; e < EPT; ++e) old[e] = dst.load_old(b, colc, Pos(t, TPS * e, TPS, L));
-  if (act) {
-#pragma unroll
-    for (int e = 0; e < EPT; ++e) dst.store(b, col, Pos(t, TPS * e, TPS, L), v[e], old[e]);
-  }
+  for (int e = 0; e < EPT; ++e) old[e] = dst.load_old(b, colc, Pos(ts, TPS * e, TPS, L));
+  if (act) store_line<TPS, L>(dst, b, col, ts, v, old);
 }
 
 // Persistent, software-pipelined variant of k_col: gridDim.x workgroups (a
@@ -391,8 +484,6 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
     k_col_pipe(Src src, Dst dst, const cx<T>* __restrict__ tw, int ncols, int ntiles, long long nitems) {
   constexpr int EPT = PlanInfo<L, V>::EPT, TPS = PlanInfo<L, V>::TPS;
   extern __shared__ __align__(16) unsigned char col_lds_raw[];  // TwLds<T, L, C, V>::bytes
-  cx<T>* const lds = reinterpret_cast<cx<T>*>(col_lds_raw);
-  cx<T>* const twl = lds + L * C;
   const int c = threadIdx.x % C, t = threadIdx.x / C;
   long long w, hi;
   int step;
@@ -406,7 +497,7 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
     for (int e = 0; e < EPT; ++e) v[e] = src.load(b, colc, Pos(tq, TPS * e, TPS, L));
   };
   fetch(w, t, nx);
-  const ColTw<T, L, C, V> ft(tw, twl);
+  const ColTw<T, L, C, V> ft(tw, col_lds_raw);
   for (; w < hi; w += step) {
     // per-element positions recomputed each item (an empty asm statement
     // hides that they do not change), not held in registers across the loop
@@ -418,17 +509,14 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
     if (w + step < hi) fetch(w + step, tq, nx);
     // every stage exchange of the previous item ended with a barrier after
     // its last LDS read, so the first exchange of this one may write
-    ft.template exec<INV>(v, lds + c, C, t);
+    ft.template exec<INV>(v, c, t);
     const int b = __builtin_amdgcn_readfirstlane((int)(w / ntiles)),
               col = __builtin_amdgcn_readfirstlane((int)(w % ntiles)) * C + c;
     const int colc = col < ncols ? col : ncols - 1;
     cx<T> old[EPT];
 #pragma unroll
     for (int e = 0; e < EPT; ++e) old[e] = dst.load_old(b, colc, Pos(tq, TPS * e, TPS, L));
-    if (col < ncols) {
-#pragma unroll
-      for (int e = 0; e < EPT; ++e) dst.store(b, col, Pos(tq, TPS * e, TPS, L), v[e], old[e]);
-    }
+    if (col < ncols) store_line<TPS, L>(dst, b, col, tq, v, old);
   }
 }
 
@@ -452,32 +540,36 @@ struct MultiPow {
   cx<T>* out[3];
   int pw[3];
   int no;
+  int nt = 0;
+  void stream(int C) {
+    nt = 1;
+    for (int o = 0; o < no; ++o) nt &= streams(out[o], C, dst.sb, dst.sp, sizeof(cx<T>));
+  }
   __device__ __forceinline__ cx<T> load(int o, int b, int col, Pos pos) const {
     SrcPadPow<T> s = src;
     s.pw = o == 0 ? pw[0] : (o == 1 ? pw[1] : pw[2]);
     return s.load(b, col, pos);
   }
+  template <bool NT = false>
   __device__ __forceinline__ void store(int o, int b, int col, Pos pos, cx<T> v) const {
     DstPlain<T> d = dst;
     d.p = o == 0 ? out[0] : (o == 1 ? out[1] : out[2]);
-    d.store(b, col, pos, v, v);
+    d.template store<NT>(b, col, pos, v, v);
   }
 };
 
 template <typename T, int L, bool INV, int C, int V, class M>
-__global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
+__global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS), (col_waves<T, L, C, V>()))
     k_col_multi(M a, const cx<T>* __restrict__ tw, int ncols) {
   constexpr int EPT = PlanInfo<L, V>::EPT, TPS = PlanInfo<L, V>::TPS;
   extern __shared__ __align__(16) unsigned char col_lds_raw[];  // TwLds<T, L, C, V>::bytes
-  cx<T>* const lds = reinterpret_cast<cx<T>*>(col_lds_raw);
-  cx<T>* const twl = lds + L * C;
   const int c = threadIdx.x % C, t = threadIdx.x / C;
   int tile, b;
   xcd_tile(tile, b);
   const int col = tile * C + c;
   const bool act = col < ncols;
   const int colc = act ? col : ncols - 1;
-  const ColTw<T, L, C, V> ft(tw, twl);
+  const ColTw<T, L, C, V> ft(tw, col_lds_raw);
 #pragma unroll 1
   for (int o = 0; o < a.no; ++o) {
     // the line position and column pass through an empty asm statement per
@@ -491,10 +583,16 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
     for (int e = 0; e < EPT; ++e) v[e] = a.load(o, b, cq, Pos(tq, TPS * e, TPS, L));
     // the previous output's last exchange ended with a barrier after its
     // last LDS read, so this transform's first exchange may write
-    ft.template exec<INV>(v, lds + c, C, t);
+    ft.template exec<INV>(v, c, tq);
+    asm volatile("" : "+v"(tq), "+v"(colq));
     if (act) {
+      if (a.nt) {
 #pragma unroll
-      for (int e = 0; e < EPT; ++e) a.store(o, b, colq, Pos(tq, TPS * e, TPS, L), v[e]);
+        for (int e = 0; e < EPT; ++e) a.template store<true>(o, b, colq, Pos(tq, TPS * e, TPS, L), v[e]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < EPT; ++e) a.store(o, b, colq, Pos(tq, TPS * e, TPS, L), v[e]);
+      }
     }
   }
 }
@@ -534,6 +632,10 @@ struct TurnArgs {
   long long osb, osp;
   int nb;            // line sets of one array; further arrays sq apart
   long long sq, osq;
+  int nt = 0;
+  void stream(int C) {
+    nt = streams(out, C, osb, osp, sizeof(cx<T>)) && ((unsigned long long)osq * sizeof(cx<T>)) % 128 == 0;
+  }
   __device__ __forceinline__ const cx<T>* from(int b) const {
     const int q = b / nb;
     return src + (long long)q * sq + (long long)(b - q * nb) * sb;
@@ -554,12 +656,10 @@ __device__ __forceinline__ bool turn_zero(int t, int c, int W, int L) {
 }
 
 template <typename T, int L, int C, int V = 0>
-__global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
+__global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS), (col_waves<T, L, C, V>()))
     k_col_turn(TurnArgs<T> a, const cx<T>* __restrict__ tw, int ncols) {
   constexpr int EPT = PlanInfo<L, V>::EPT, TPS = PlanInfo<L, V>::TPS;
   extern __shared__ __align__(16) unsigned char col_lds_raw[];  // TwLds<T, L, C, V>::bytes
-  cx<T>* const lds = reinterpret_cast<cx<T>*>(col_lds_raw);
-  cx<T>* const twl = lds + L * C;
   const int c = threadIdx.x % C, t = threadIdx.x / C;
   int tile, b;
   xcd_tile(tile, b);
@@ -571,22 +671,29 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
   cx<T> x[EPT];
 #pragma unroll
   for (int e = 0; e < EPT; ++e) x[e] = *line_at(from, a.sp, colc, t, TPS * e);
-  const ColTw<T, L, C, V> ft(tw, twl);
-  ft.template exec<false>(x, lds + c, C, t);
+  const ColTw<T, L, C, V> ft(tw, col_lds_raw);
+  ft.template exec<false>(x, c, t);
   const bool nyqc = colc == nh;
 #pragma unroll
   for (int e = 0; e < EPT; ++e) {
     // dropped positions and the Nyquist mode (index n/2 is position n/2 = L/3)
     const bool zero = turn_zero(t, TPS * e, TPS, L) | nyqc;
     const cx<T> o = x[e] * a.fscale;  // the n-grid value
-    x[e] = zero ? mk(T(0), T(0)) : o * a.iscale;
+    x[e] = or_zero(!zero, o * a.iscale);
   }
   __syncthreads();  // the forward transform's exchange reads are done
-  ft.template exec<true>(x, lds + c, C, t);
+  int ti = t;  // LDS and line addresses formed again, not held in registers since the forward transform
+  asm volatile("" : "+v"(ti));
+  ft.template exec<true>(x, c, ti);
   if (act) {
     cx<T>* const to = a.to(b);
+    if (a.nt) {
 #pragma unroll
-    for (int e = 0; e < EPT; ++e) *line_at(to, a.osp, col, t, TPS * e) = x[e];
+      for (int e = 0; e < EPT; ++e) put<true>(line_at(to, a.osp, col, ti, TPS * e), x[e]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < EPT; ++e) *line_at(to, a.osp, col, ti, TPS * e) = x[e];
+    }
   }
 }
 
@@ -596,8 +703,6 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
     k_col_turn_pipe(TurnArgs<T> a, const cx<T>* __restrict__ tw, int ncols, int ntiles, long long nitems) {
   constexpr int EPT = PlanInfo<L, V>::EPT, TPS = PlanInfo<L, V>::TPS;
   extern __shared__ __align__(16) unsigned char col_lds_raw[];  // TwLds<T, L, C, V>::bytes
-  cx<T>* const lds = reinterpret_cast<cx<T>*>(col_lds_raw);
-  cx<T>* const twl = lds + L * C;
   const int c = threadIdx.x % C, t = threadIdx.x / C;
   const int nh = a.n >> 1;
   long long w, hi;
@@ -613,7 +718,7 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
     for (int e = 0; e < EPT; ++e) v[e] = *line_at(from, a.sp, colc, tq, TPS * e);
   };
   fetch(w, t, nx);
-  const ColTw<T, L, C, V> ft(tw, twl);
+  const ColTw<T, L, C, V> ft(tw, col_lds_raw);
   for (; w < hi; w += step) {
     int tq = t;  // recomputed per item (see k_col_pipe)
     asm volatile("" : "+v"(tq));
@@ -624,20 +729,25 @@ __global__ void __launch_bounds__((C * PlanInfo<L, V>::TPS))
     const int b = __builtin_amdgcn_readfirstlane((int)(w / ntiles)),
               col = __builtin_amdgcn_readfirstlane((int)(w % ntiles)) * C + c;
     const int colc = col < ncols ? col : ncols - 1;
-    ft.template exec<false>(x, lds + c, C, t);
+    ft.template exec<false>(x, c, t);
     const bool nyqc = colc == nh;
 #pragma unroll
     for (int e = 0; e < EPT; ++e) {
       const bool zero = turn_zero(tq, TPS * e, TPS, L) | nyqc;
       const cx<T> o = x[e] * a.fscale;
-      x[e] = zero ? mk(T(0), T(0)) : o * a.iscale;
+      x[e] = or_zero(!zero, o * a.iscale);
     }
     __syncthreads();  // the forward transform's exchange reads are done
-    ft.template exec<true>(x, lds + c, C, t);
+    ft.template exec<true>(x, c, t);
     if (col < ncols) {
       cx<T>* const to = a.to(b);
+      if (a.nt) {
 #pragma unroll
-      for (int e = 0; e < EPT; ++e) *line_at(to, a.osp, col, tq, TPS * e) = x[e];
+        for (int e = 0; e < EPT; ++e) put<true>(line_at(to, a.osp, col, tq, TPS * e), x[e]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < EPT; ++e) *line_at(to, a.osp, col, tq, TPS * e) = x[e];
+      }
     }
   }
 }
@@ -681,6 +791,7 @@ template <typename T, int L, int C, bool INV, bool PIPE, int V, class Src, class
 void launch_col_LC(Ctx& c, Src s, Dst d, int ncols, int nbatch, const char* name, double bytes) {
   const dim3 block(C * PlanInfo<L, V>::TPS);
   const int ntiles = (ncols + C - 1) / C;
+  set_stream(d, C);
   LaunchScope ls(c, name, bytes);
   constexpr size_t dyn = TwLds<T, L, C, V>::bytes;
   if constexpr (PIPE) {
@@ -867,8 +978,14 @@ void launch_col_pad(Ctx& c, int L, Src s, Dst d, int ncols, int nbatch, const ch
   }
 }
 
+// the y stage of the Hessian rows of `planes` x-planes (lpt_engine.hip)
+template <typename T>
+void launch_hess_y(Ctx& c, int m, const SrcHessY<T>& s, const DstHessY<T>& d, int ncols, int planes, const char* name,
+                   double bytes);
+
 template <typename T, int L, int C, bool PIPE, int V>
-void launch_turn_LC(Ctx& c, const TurnArgs<T>& a, int ncols, int nbatch, const char* name, double bytes) {
+void launch_turn_LC(Ctx& c, TurnArgs<T> a, int ncols, int nbatch, const char* name, double bytes) {
+  set_stream(a, C);
   const dim3 block(C * PlanInfo<L, V>::TPS);
   const int ntiles = (ncols + C - 1) / C;
   LaunchScope ls(c, name, bytes);
@@ -943,7 +1060,8 @@ void launch_turn(Ctx& c, int L, const TurnArgs<T>& a, int ncols, int nbatch, con
 }
 
 template <typename T, int L, int C, bool INV, int V, class M>
-void launch_multi_LC(Ctx& c, const M& a, int ncols, int nbatch, const char* name, double bytes) {
+void launch_multi_LC(Ctx& c, M a, int ncols, int nbatch, const char* name, double bytes) {
+  set_stream(a, C);
   const dim3 block(C * PlanInfo<L, V>::TPS);
   const int ntiles = (ncols + C - 1) / C;
   LaunchScope ls(c, name, bytes);

@@ -34,6 +34,16 @@
 
 namespace mfx {
 
+template <typename T>
+void launch_hess_y(Ctx& c, int m, const SrcHessY<T>& s, const DstHessY<T>& d, int ncols, int planes, const char* name,
+                   double bytes) {
+  launch_col_pad<T, true>(c, m, s, d, ncols, 6 * planes, name, bytes);
+}
+template void launch_hess_y<float>(Ctx&, int, const SrcHessY<float>&, const DstHessY<float>&, int, int, const char*,
+                                   double);
+template void launch_hess_y<double>(Ctx&, int, const SrcHessY<double>&, const DstHessY<double>&, int, int, const char*,
+                                    double);
+
 // ------------------------------------------------------------------ z stage
 // compile-time loop: f(std::integral_constant<int, O>) for O = B .. N-1
 template <int B, int N, class F>
@@ -565,7 +575,7 @@ struct Engine {
     // from X_0, Yx, Yxy from X_1, Yxx from X_2
     SrcHessY<T> s{{T1[0], T1[1], T1[2]}, (long long)n * hp, hp, n, kfac};
     DstHessY<T> d{{Y[0], Y[2], Y[5], Y[1], Y[4], Y[3]}, (long long)m * hp, hp};
-    launch_col_pad<T, true>(c, m, s, d, l.h, 6 * m, "lpt_y_inv", 3 * bT1 + 6 * bT2);
+    launch_hess_y<T>(c, m, s, d, l.h, m, "lpt_y_inv", 3 * bT1 + 6 * bT2);
   }
 
   // How many of `cnt` equal arrays of `bytes` go through a chain of passes in one

@@ -187,6 +187,7 @@ void launch_col_any(Ctx& c, int L, Src s, Dst d, int ncols, int nbatch, const ch
   if (m.ok) {
     auto k = k_mix_col<T, INV, Src, Dst>;
     col_lds_prep(c, k, m.lds);
+    set_stream(d, 1 << m.lc);
     LaunchScope ls(c, name, bytes);
     hipLaunchKernelGGL(k, dim3((ncols + (1 << m.lc) - 1) >> m.lc, nbatch), dim3(m.block), m.lds, c.stream, s, d,
                        c.twiddles<T>(L), ncols, m.p, m.lc, m.nthr);
@@ -212,7 +213,9 @@ void launch_turn_any(Ctx& c, int L, const TurnArgs<T>& a, int ncols, int nbatch,
   auto k = k_mix_turn<T, TurnArgs<T>>;
   col_lds_prep(c, k, m.lds);
   LaunchScope ls(c, name, bytes);
-  hipLaunchKernelGGL(k, dim3((ncols + (1 << m.lc) - 1) >> m.lc, nbatch), dim3(m.block), m.lds, c.stream, a,
+  TurnArgs<T> ta = a;
+  set_stream(ta, 1 << m.lc);
+  hipLaunchKernelGGL(k, dim3((ncols + (1 << m.lc) - 1) >> m.lc, nbatch), dim3(m.block), m.lds, c.stream, ta,
                      c.twiddles<T>(L), ncols, m.p, m.lc, m.nthr);
   check_launch(name);
 }

@@ -166,8 +166,6 @@ __global__ void __launch_bounds__((C * PlanInfo<L, 0>::TPS))
     k_col_fwd_mul_inv(Src src, Dst dst, Mul mul, const cx<T>* __restrict__ tw, int ncols) {
   constexpr int EPT = PlanInfo<L, 0>::EPT, TPS = PlanInfo<L, 0>::TPS;
   extern __shared__ __align__(16) unsigned char col_lds_raw[];  // TwLds<T, L, C, 0>::bytes
-  cx<T>* const lds = reinterpret_cast<cx<T>*>(col_lds_raw);
-  cx<T>* const twl = lds + L * C;
   const int c = threadIdx.x % C, t = threadIdx.x / C;
   int tile, b;
   xcd_tile(tile, b);
@@ -177,14 +175,14 @@ __global__ void __launch_bounds__((C * PlanInfo<L, 0>::TPS))
   cx<T> v[EPT];
 #pragma unroll
   for (int e = 0; e < EPT; ++e) v[e] = src.load(b, colc, Pos(t, TPS * e, TPS, L));
-  const ColTw<T, L, C, 0> ft(tw, twl);
-  ft.template exec<false>(v, lds + c, C, t);
+  const ColTw<T, L, C, 0> ft(tw, col_lds_raw);
+  ft.template exec<false>(v, c, t);
 #pragma unroll
   for (int e = 0; e < EPT; ++e) v[e] = cmul(v[e], mul(b, colc, t + TPS * e));
-  ft.template exec<true>(v, lds + c, C, t);
+  ft.template exec<true>(v, c, t);
   if (act) {
-#pragma unroll
-    for (int e = 0; e < EPT; ++e) dst.store(b, col, Pos(t, TPS * e, TPS, L), v[e], mk(T(0), T(0)));
+    const cx<T> none[EPT] = {};
+    store_line<TPS, L>(dst, b, col, t, v, none);
   }
 }
 
@@ -195,6 +193,7 @@ void launch_fmi_L(Ctx& c, Src s, Dst d, Mul m, int ncols, int nbatch, const char
   constexpr size_t dyn = TwLds<T, L, C, 0>::bytes;
   auto k = k_col_fwd_mul_inv<T, L, C, Src, Dst, Mul>;
   col_lds_prep(c, k, dyn);
+  set_stream(d, C);
   LaunchScope ls(c, name, bytes);
   hipLaunchKernelGGL(k, dim3((ncols + C - 1) / C, nbatch), block, dyn, c.stream, s, d, m, c.twiddles<T>(L), ncols);
   check_launch(name);
