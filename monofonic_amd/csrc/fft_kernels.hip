@@ -270,7 +270,7 @@ void autotune_columns(Ctx& c, int L) {
         // at a padded length the row-strided inverse pass is the y stage of the
         // Hessian rows: six outputs of three sources, as many planes as the block
         // holds.  An in-place pass prefers other variants: 384-line FP64 1.94 ms of
-        // its choice against 1.00, 768-line FP32 4.72 against 4.15 (two fields)
+        // its choice against 1.00 to 1.35, 768-line FP32 4.72 against 4.15 (two fields)
         const int planes = (int)((long long)nb * L / (3ll * nn + 6ll * L));
         if (padded && inv && cls == 0 && planes > 0) {
           const long long xs = (long long)planes * nn * pitch, ys = (long long)planes * L * pitch;

@@ -21,8 +21,8 @@ constexpr int CU_LDS = 160 * 1024;  // LDS of a compute unit
 // Tile widths of a column pass of length L (plan variant V): C, the widest
 // tile (at most 16 columns) whose exchange area fits 64 KiB of LDS, and CW =
 // 2C where C < 16 and a tile of 2C columns still fits one workgroup (1024
-// threads, 160 KiB of LDS with its twiddle table; one workgroup per CU), else
-// 0.  Wider tiles read longer runs of each line (2C complex values).
+// threads; exchanged in two parts, TwLds), else 0.  Wider tiles read longer runs
+// of each line (2C complex values).
 template <typename T, int L, int V = 0>
 struct ColCfg {
   static constexpr int TPS = PlanInfo<L, V>::TPS;
@@ -269,7 +269,7 @@ struct SrcPadPow {
 // the powers 0, 1 of X_1, 5 is X_2.  The outputs of a plane that share their
 // source follow one another on an XCD, a plane (1.1 MB at n = 512, FP32) apart.
 // One launch instead of six: 96^3 FP64 75 -> 47 us for a field, 256^3 FP64 0.82 ->
-// 0.67 ms, 512^3 FP32 2.80 -> 2.75 ms.
+// 0.67 ms, 512^3 FP32 2.80 -> 2.75 ms (2.00 with streaming stores).
 template <typename T>
 struct SrcHessY {
   const cx<T>* x[3];
@@ -1092,8 +1092,8 @@ void launch_multi_LV(Ctx& c, int v, const M& a, int ncols, int nbatch, const cha
 
 // at the tile width tuned for (L, T, INV) and the stride class of line
 // stride sp; the multi-output kernel has no pipelined form and always runs
-// plan 0 (with the second plan the three-output Hessian pass compiles to 179
-// instead of 95 VGPRs, two waves per SIMD instead of five)
+// plan 0 (with the second plan the three-output Hessian pass compiled to 179
+// instead of 95 VGPRs, two waves per SIMD instead of five; plan 0 now takes 80)
 template <typename T, int L, bool INV, class M>
 void launch_multi_L(Ctx& c, const M& a, long long sp, int ncols, int nbatch, const char* name, double bytes) {
   const int v = c.col_tile(L, (int)sizeof(T), INV, ColCfg<T, L>::C, stride_class(sp, (int)sizeof(cx<T>)));
