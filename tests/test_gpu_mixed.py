@@ -82,3 +82,21 @@ def test_lpt_streamed_request_keeps_the_sequence(ctx, orc, n):
     conv.lpt_sources(phi, phi2, phi3, tuple(A3), order=3)
     for g, s in zip((phi2, phi3, *A3), seq):
         assert rel_rms(g.kdata(), s) < 1e-12
+
+
+@pytest.mark.parametrize("shape", [(20, 16, 40), (150, 16, 32), (35, 20, 16), (70, 16, 300)])
+@pytest.mark.parametrize("prec", ["float", "double"])
+def test_constant_field_has_one_mode(ctx, shape, prec):
+    """the butterflies cancel a line's mean exactly, with rounded constants too
+    (lengths of two and more mixed-radix stages; single primes run other kernels)"""
+    import monofonic_amd as M
+    print(f"constant field {shape} {prec}", flush=True)
+    a = np.zeros(shape[:2] + (shape[2] + 2,))
+    a[:, :, :shape[2]] = 1.0
+    g = M.Grid_FFT(ctx, shape, (100.0, 100.0, 100.0), prec)
+    g.upload(a)
+    g.FourierTransformForward()
+    k = g.kdata().copy()
+    assert abs(k[0, 0, 0] / np.sqrt(np.prod(shape)) - 1) < 1e-6
+    k[0, 0, 0] = 0
+    assert not k.any()
