@@ -79,6 +79,14 @@ bool mix_plan(int L, int rmax, int fixed_last, MixPlan& p) {
         r[n - 1] = t;
         break;
       }
+    // an even radix first where there is one: it keeps a line's mean out of its
+    // longest waves without the more costly odd form (mix_first_bf)
+    if (r[0] % 2)
+      for (int i = 1; i < n; ++i)
+        if (r[i] % 2 == 0) {
+          for (int q = i; q > 0; --q) std::swap(r[q], r[q - 1]);
+          break;
+        }
   }
   p = MixPlan{};
   p.L = L;
