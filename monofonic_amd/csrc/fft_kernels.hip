@@ -188,15 +188,22 @@ void conv2(Ctx& c, const cx<T>* fa, const MultSpec& ma, const cx<T>* fb, const M
     DstPlain<T> d2{t2s[o], (long long)m * hp, hp, T(1)};
     launch_col<T, true>(c, m, s2, d2, h, m, "conv_p2_yinv", bT1 + bT2);
   }
-  // P3: z c2r x2, product, r2c, truncate (in place into T2a)
-  launch_row_prod<T>(c, m / 2, T2a, T2b, hp, h, T2a, hp, h, (long long)m * m, "conv_p3_zprod", 3 * bT2);
+  // P3: z c2r x2, product, r2c, truncate (in place into T2a); T1b is free from here on
+  T* const mean = reinterpret_cast<T*>(T1b);
+  const bool less_mean = launch_row_mean<T>(c, m / 2, T2a, T2b, hp, h, (long long)m * m, mean, "conv_p3_mean");
+  launch_row_prod<T>(c, m / 2, T2a, T2b, hp, h, T2a, hp, h, (long long)m * m, less_mean ? mean : nullptr,
+                     "conv_p3_zprod", 3 * bT2);
   // P4: y-forward truncation, T2a [x][y][kz] -> T1a [x][j][kz]
   launch_col<T, false>(c, m, SrcPlain<T>{T2a, (long long)m * hp, hp}, DstTrunc<T>{T1a, (long long)n * hp, hp, n}, h,
                        m, "conv_p4_yfwd", bT2 + bT1);
   // P5: x-forward truncation + op into out [i][j][kz]
   DstTruncOp<T> d5{{out}, n, HN, (long long)n * HN, n, op, T(opfac), s_out, 0, kfac};
-  launch_col<T, false>(c, m, SrcPlain<T>{T1a, hp, (long long)n * hp}, d5, h, n, "conv_p5_xfwd",
-                       bT1 + (op == OP_ASSIGN ? bN : 2 * bN));
+  const SrcPlain<T> s5{T1a, hp, (long long)n * hp};
+  const double b5 = bT1 + (op == OP_ASSIGN ? bN : 2 * bN);
+  if (less_mean)
+    launch_col_any<T, false>(c, m, s5, DstTruncOpMean<T>{d5, mean, T((double)m * m * m)}, h, n, "conv_p5_xfwd", b5);
+  else
+    launch_col<T, false>(c, m, s5, d5, h, n, "conv_p5_xfwd", b5);
 }
 
 // ------------------------------------------------------------------ autotuning

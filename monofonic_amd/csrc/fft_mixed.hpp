@@ -752,11 +752,60 @@ __device__ __forceinline__ cx<T> mix_pmul(cx<T> a, cx<T> b) {
   return mk(a.x * b.x, a.y * b.y);
 }
 
-// P3: c2r of two half spectra, pointwise product, r2c
+// The mean of a product of the m x m rows of two half spectra, from MIX_MEAN_ROWS of
+// them on a lattice: a row's mean is Re(a_0) Re(b_0) + 2 sum Re(a_k conj(b_k)).  One
+// workgroup, two rows a wave, whose loads are all in flight together.
+constexpr int MIX_MEAN_ROWS = 32;
+template <typename T>
+__global__ void __launch_bounds__(1024)
+    k_mix_mean(const cx<T>* a, const cx<T>* b, long long spitch, int hin, int m, T* mean) {
+  __shared__ T part[16];
+  constexpr int N = MIX_MEAN_ROWS, U = 4;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const cx<T>*u[N / 16], *v[N / 16];
+#pragma unroll
+  for (int q = 0; q < N / 16; ++q) {
+    const int s = wave + 16 * q;
+    const long long row = ((long long)(s * m / N) * m + (19 * s) % N * m / N) * spitch;
+    u[q] = a + row;
+    v[q] = b + row;
+  }
+  T sum = 0;
+  for (int k0 = lane; k0 < hin; k0 += 64 * U) {
+    cx<T> x[N / 16][U], y[N / 16][U];
+#pragma unroll
+    for (int q = 0; q < N / 16; ++q)
+#pragma unroll
+      for (int e = 0; e < U; ++e) {
+        const int k = k0 + 64 * e < hin ? k0 + 64 * e : hin - 1;
+        x[q][e] = u[q][k];
+        y[q][e] = v[q][k];
+      }
+#pragma unroll
+    for (int q = 0; q < N / 16; ++q)
+#pragma unroll
+      for (int e = 0; e < U; ++e) {
+        const int k = k0 + 64 * e;
+        const T re = x[q][e].x * y[q][e].x, im = x[q][e].y * y[q][e].y;
+        sum += pick(k == 0, re, pick(k < hin, T(2) * (re + im), T(0)));
+      }
+  }
+  sum = sum * (T(1) / T(N));
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) sum += __shfl_down(sum, d);
+  if (lane == 0) part[wave] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 16; ++w) sum += part[w];
+    *mean = sum;
+  }
+}
+
+// P3: c2r of two half spectra, pointwise product less *mean (if not null), r2c
 template <typename T>
 __global__ void __launch_bounds__(512)
     k_mix_prod(const cx<T>* a, const cx<T>* b, long long spitch, cx<T>* dst, long long dpitch, int hout,
-               MixRowArgs ra, const cx<T>* __restrict__ tw) {
+               const T* mean, MixRowArgs ra, const cx<T>* __restrict__ tw) {
   extern __shared__ __align__(16) unsigned char col_lds_raw[];
   const MixRow<T> r(ra, reinterpret_cast<cx<T>*>(col_lds_raw));
   const MixZ<T> z{r, ra.p};
@@ -769,6 +818,11 @@ __global__ void __launch_bounds__(512)
   z.c2r(v, wb, MixOne<T>{});
 #pragma unroll
   for (int q = 0; q < MixZ<T>::S; ++q) u[q] = mix_pmul(u[q], v[q]);
+  if (mean) {
+    const T c = *mean;
+#pragma unroll
+    for (int q = 0; q < MixZ<T>::S; ++q) u[q] = u[q] - mk(c, c);
+  }
   z.r2c(u, dst + r.ra * dpitch, dst + r.rb * dpitch, hout);
 }
 

@@ -361,6 +361,18 @@ struct DstTruncOp {
   }
 };
 
+// DstTruncOp of one array for a product transformed without (nearly all of) its
+// mean: *mean times the number of points goes back to the k = 0 mode
+template <typename T>
+struct DstTruncOpMean : DstTruncOp<T> {
+  const T* mean;
+  T count;
+  __device__ __forceinline__ void store(int b, int col, Pos pos, cx<T> v, cx<T> prev) const {
+    const bool dc = ((int)pos == 0) & (b == 0) & (col == 0);
+    DstTruncOp<T>::store(b, col, pos, mk(v.x + pick(dc, *mean * count, T(0)), v.y), prev);
+  }
+};
+
 // The last (x) pass of the noise's forward transform writing phi(1) instead
 // of the k-space noise (ic_generator.cc:341-346,450-457): each transformed
 // value is scaled as the plain pass would store it (rounded to T) and turned
@@ -942,7 +954,12 @@ void launch_row_c2r_part_any(Ctx& c, int K, const cx<T>* src, long long spitch, 
                              long long nrows, T scale, double lunit, double qoff, const char* name, double bytes);
 template <typename T>
 void launch_row_prod_any(Ctx& c, int K, const cx<T>* a, const cx<T>* b, long long spitch, int hin, cx<T>* dst,
-                         long long dpitch, int hout, long long nrows, const char* name, double bytes);
+                         long long dpitch, int hout, long long nrows, const T* mean, const char* name, double bytes);
+// the mean of such a product into *mean, where launch_row_prod is to take it off
+// (false: it is not)
+template <typename T>
+bool launch_row_mean(Ctx& c, int K, const cx<T>* a, const cx<T>* b, long long spitch, int hin, long long nrows,
+                     T* mean, const char* name);
 
 template <typename T, bool INV, class Src, class Dst>
 void launch_col(Ctx& c, int L, Src s, Dst d, int ncols, int nbatch, const char* name, double bytes) {
@@ -1375,14 +1392,16 @@ void launch_row_c2r_part(Ctx& c, int K, const cx<T>* src, long long spitch, int 
 #undef MFX_CASE
 }
 
+// mean: what launch_row_mean gave, or null
 template <typename T>
 void launch_row_prod(Ctx& c, int K, const cx<T>* a, const cx<T>* b, long long spitch, int hin, cx<T>* dst,
-                     long long dpitch, int hout, long long nrows, const char* name, double bytes) {
+                     long long dpitch, int hout, long long nrows, const T* mean, const char* name, double bytes) {
 #define MFX_CASE(KK)                                                                                \
   case KK:                                                                                          \
     launch_row_prod_K<T, KK>(c, a, b, spitch, hin, dst, dpitch, hout, nrows, name, bytes);        \
     return;
-  MFX_ROW_SWITCH(K, MFX_CASE, launch_row_prod_any<T>(c, K, a, b, spitch, hin, dst, dpitch, hout, nrows, name, bytes))
+  MFX_ROW_SWITCH(K, MFX_CASE, 
+                 launch_row_prod_any<T>(c, K, a, b, spitch, hin, dst, dpitch, hout, nrows, mean, name, bytes))
 #undef MFX_CASE
 }
 
