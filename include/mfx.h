@@ -208,9 +208,12 @@ int mfx_lpt_sources(mfx_conv *cv, mfx_grid *phi, mfx_grid *phi2, mfx_grid *phi3,
  * mfx_conv_lpt_path reports it (MFX_LPT_AUTO while not yet made).
  * Grid sizes without tuned z stages (7-smooth multiples of 4 other than
  * 16..1024 of the forms 2^k and 3*2^k with a tuned 3n/2) have the stored path
- * only: where its workspace takes at most a third of the free memory, or, set
- * to stored, leaves 8 GiB free.  Else, and set to streamed, such a size runs
- * the convolve sequence. */
+ * only: where its workspace takes at most a third of the free memory and leaves
+ * half of the device free, or, set to stored, leaves 8 GiB free.  Else, and set to
+ * streamed, such a size runs the convolve sequence.  When an allocation of the
+ * library on this context finds no memory left, such workspaces are given back,
+ * but for those that a captured graph uses, and their convolvers run the sequence
+ * until the path is set again (an allocation outside the library gets none back). */
 #define MFX_LPT_AUTO 0
 #define MFX_LPT_STREAMED 1
 #define MFX_LPT_STORED 2

@@ -69,8 +69,7 @@ const cx<T>* Ctx::twiddles(int L) {
     h[n].x = (T)cosl(a);
     h[n].y = (T)(-sinl(a));
   }
-  void* d = nullptr;
-  MFX_HIP(hipMalloc(&d, sizeof(cx<T>) * L));
+  void* d = alloc(sizeof(cx<T>) * L);
   MFX_HIP(hipMemcpy(d, h.data(), sizeof(cx<T>) * L, hipMemcpyHostToDevice));
   tw[key] = d;
   return reinterpret_cast<const cx<T>*>(d);
@@ -90,8 +89,29 @@ int Ctx::num_cus() {
 void* Ctx::alloc(size_t bytes) {
   void* p = nullptr;
   if (bytes == 0) bytes = 16;
-  MFX_HIP(hipMalloc(&p, bytes));
+  hipError_t e = hipMalloc(&p, bytes);
+  if (e == hipErrorOutOfMemory && release_spare()) {
+    (void)hipGetLastError();
+    e = hipMalloc(&p, bytes);
+  }
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    throw Error(2, "hipMalloc of " + std::to_string(bytes) + " bytes failed: " + hipGetErrorString(e));
+  }
   return p;
+}
+bool Ctx::capturing() {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+bool Ctx::release_spare() {
+  if (spare.empty() || capturing()) return false;
+  MFX_HIP(hipStreamSynchronize(stream));
+  bool any = false;
+  for (auto& s : spare) any |= s.second();
+  return any;
 }
 void Ctx::release(void* p) {
   if (p) MFX_HIP(hipFree(p));
@@ -129,6 +149,9 @@ struct mfx_conv {
   int lpt_path = MFX_LPT_AUTO;  // requested 3LPT path
   int lpt_chosen = MFX_LPT_AUTO;  // path the 3LPT workspace was reserved for
   int lpt_refused = 0;  // lowest LPT order whose engine workspace did not fit (0: none)
+  bool lpt_busy = false;      // its sources are being issued
+  bool lpt_captured = false;  // a captured graph holds the workspace's address
+  std::vector<void*> lpt_old;  // outgrown workspaces that captured graphs hold
   mfx_grid* fbuf = nullptr;  // convolve3 intermediate (convolution.hh:469)
 };
 
@@ -631,7 +654,9 @@ int mfx_conv_destroy(mfx_conv* cv) {
     if (!cv) return;
     MFX_HIP(hipStreamSynchronize(cv->ctx->c.stream));
     cv->ctx->c.release(cv->ws);
+    cv->ctx->c.spare.erase(cv);
     cv->ctx->c.release(cv->lpt_ws);
+    for (void* p : cv->lpt_old) cv->ctx->c.release(p);
     if (cv->fbuf) {
       cv->ctx->c.release(cv->fbuf->d);
       delete cv->fbuf;
@@ -889,15 +914,25 @@ static int lpt_choose(mfx_conv* cv) {
   return st + headroom <= fr + cv->lpt_bytes ? MFX_LPT_STORED : MFX_LPT_STREAMED;
 }
 
+static void lpt_free(mfx_conv* cv) {
+  MFX_HIP(hipStreamSynchronize(cv->ctx->c.stream));
+  cv->ctx->c.release(cv->lpt_ws);
+  cv->lpt_ws = nullptr;
+  cv->lpt_bytes = 0;
+}
+
 // workspace of the fused engine for LPT order `order` (grown on demand)
 static void lpt_reserve(mfx_conv* cv, int order) {
   if (order > 2 && cv->lpt_chosen == MFX_LPT_AUTO) cv->lpt_chosen = lpt_choose(cv);
   const size_t need = lpt_workspace_bytes(cv->n, cv->prec, order, cv->lpt_chosen == MFX_LPT_STORED);
   if (cv->lpt_bytes < need) {
-    MFX_HIP(hipStreamSynchronize(cv->ctx->c.stream));
-    cv->ctx->c.release(cv->lpt_ws);
+    if (cv->lpt_captured)
+      cv->lpt_old.push_back(cv->lpt_ws);
+    else
+      lpt_free(cv);
     cv->lpt_ws = nullptr;
     cv->lpt_bytes = 0;
+    cv->lpt_captured = false;
     cv->lpt_ws = cv->ctx->c.alloc(need);
     cv->lpt_bytes = need;
   }
@@ -906,11 +941,13 @@ static void lpt_reserve(mfx_conv* cv, int order) {
 // Whether the fused engine runs this convolver's sources at LPT order `order`,
 // its workspace reserved: always at grid sizes with tuned z stages; at the
 // other sizes it supports (the mixed-radix stages: 2LPT and stored 3LPT) where
-// the workspace takes at most a third of the free device memory, so that
-// programs that hold many generators keep room for them (any room with 8 GiB to
-// spare where the caller asked for the stored path).  Otherwise the convolve
+// the workspace takes at most a third of the free device memory and leaves half of
+// the device free, so that programs that hold many generators keep room for them
+// (any room with 8 GiB to spare where the caller asked for the stored path).  Otherwise the convolve
 // sequence, whose workspace is a fraction of it.  A refusal is remembered until
-// the path is set again: the decision does not change between calls.
+// the path is set again: the decision does not change between calls.  A workspace
+// so taken is spare: when the device's memory runs out it is given back, unless
+// a captured graph holds it, and the sequence runs from then on.
 static bool lpt_engine_ready(mfx_conv* cv, int order) {
   Ctx& c = cv->ctx->c;
   if (!lpt_fused_supported(cv->n)) {
@@ -921,14 +958,25 @@ static bool lpt_engine_ready(mfx_conv* cv, int order) {
     if (cv->lpt_bytes < need) {
       size_t fr = 0, tot = 0;
       MFX_HIP(hipMemGetInfo(&fr, &tot));
-      fr += cv->lpt_bytes;
-      const bool fits = cv->lpt_path == MFX_LPT_STORED ? need + ((size_t)8 << 30) <= fr : need <= fr / 3;
+      if (!cv->lpt_captured) fr += cv->lpt_bytes;
+      const bool fits = cv->lpt_path == MFX_LPT_STORED ? need + ((size_t)8 << 30) <= fr
+                                                             : need <= fr / 3 && need + tot / 2 <= fr;
       if (!fits) {
         cv->lpt_refused = order;
         return false;
       }
     }
     if (order > 2) cv->lpt_chosen = MFX_LPT_STORED;
+    c.spare.erase(cv);
+    lpt_reserve(cv, order);
+    c.spare[cv] = [cv] {
+      if (!cv->lpt_ws || cv->lpt_busy || cv->lpt_captured) return false;
+      lpt_free(cv);
+      cv->lpt_refused = 2;
+      cv->lpt_chosen = MFX_LPT_AUTO;
+      return true;
+    };
+    return true;
   }
   lpt_reserve(cv, order);
   return true;
@@ -940,6 +988,12 @@ static void lpt_fused(mfx_conv* cv, mfx_grid* phi, mfx_grid* phi2, mfx_grid* phi
     lpt_sequence(cv, phi, phi2, phi3, A3, order);
     return;
   }
+  struct Busy {
+    mfx_conv* cv;
+    explicit Busy(mfx_conv* c) : cv(c) { cv->lpt_busy = true; }
+    ~Busy() { cv->lpt_busy = false; }
+  } busy(cv);
+  if (cv->ctx->c.capturing()) cv->lpt_captured = true;
   grid_forward(phi, true);
   phi2->space = MFX_KSPACE;
   if (order > 2) {
@@ -1544,8 +1598,8 @@ static void icgen_free(mfx_icgen* ic) {
     }
   if (ic->conv) mfx_conv_destroy(ic->conv);
   for (int w = 0; w < 12; ++w) {
-    // the baryon arrays (6..11) always have their own allocation
-    if (ic->part[w] && (w >= 6 || !ic->part_in_ws)) ic->ctx->c.release(ic->part[w]);
+    // the baryon arrays (6..11) always have their own allocations
+    if (ic->part[w] && (w >= 6 || (w == 0 && !ic->part_in_ws))) ic->ctx->c.release(ic->part[w]);
     ic->part[w] = nullptr;
   }
   if (ic->comp6 && !ic->comp6_in_ws) ic->ctx->c.release(ic->comp6);
@@ -1633,16 +1687,19 @@ extern "C" int mfx_icgen_create(mfx_ctx* c, const mfx_icgen_params* p, mfx_icgen
       // The FP64 particle arrays are written after the LPT sources are
       // complete, so with the fused engine they share its workspace (at 1024^3
       // FP32 this keeps the realisation within one GPU's HBM); they stay valid
-      // until the next run.
+      // until the next run.  Sizes that can do without the workspace keep them
+      // apart from it, so that it can be given back.
       const size_t ncell = p->n * p->n * p->n, npart = ncell * (size_t)ic->overload;
       if (ic->conv && p->use_fused_lpt && !p->own_particles && lpt_engine_ready(ic->conv, p->lpt_order)) {
-        if (ic->conv->lpt_bytes >= 6 * npart * sizeof(double)) {
+        if (lpt_fused_supported((int)p->n) && ic->conv->lpt_bytes >= 6 * npart * sizeof(double)) {
           ic->part_in_ws = true;
           for (int w = 0; w < 6; ++w) ic->part[w] = (double*)ic->conv->lpt_ws + w * npart;
         }
       }
-      if (!ic->part_in_ws)
-        for (int w = 0; w < 6; ++w) ic->part[w] = (double*)c->c.alloc(sizeof(double) * npart);
+      if (!ic->part_in_ws) {  // one allocation, of which part[0] is the start
+        ic->part[0] = (double*)c->c.alloc(6 * sizeof(double) * npart);
+        for (int w = 1; w < 6; ++w) ic->part[w] = ic->part[0] + w * npart;
+      }
       if (p->baryons)
         for (int w = 6; w < 12; ++w) ic->part[w] = (double*)c->c.alloc(sizeof(double) * npart);
       // six component grids: after the particles in the LPT workspace, else

@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <functional>
 #include <map>
 #include <stdexcept>
 #include <string>
@@ -93,8 +94,14 @@ struct Ctx {
   ~Ctx();
   template <typename T>
   const cx<T>* twiddles(int L);
+  // device memory; where there is none left, workspaces that their owners can do
+  // without (spare) are given back first
   void* alloc(size_t bytes);
   void release(void* p);
+  // owner -> gives its workspace back (false: nothing that can be)
+  std::map<const void*, std::function<bool()>> spare;
+  bool release_spare();
+  bool capturing();  // whether the stream is being captured into a graph
 };
 
 // Records events around a launch when profiling is on.  `bytes` is the
