@@ -75,11 +75,12 @@ int mfx_memcpy_h2d(mfx_ctx *c, void *dev, const void *host, size_t bytes);
  * src/grid_fft.cc:53-54).  Times the column-pass variants of lengths n and
  * 3n/2 in `precision` -- tile width (64 KiB tile, half or twice), plain or
  * persistent pipelined kernel, and for lengths 384, 768, 1024 and 1536 the
- * second radix plan -- and keeps the fastest per length and direction in
- * the context.  Tile width and kernel form never change results; the radix
+ * second radix plan -- and keeps the fastest per length, direction and use (plain
+ * grids, the passes over padded lines) in the context.  Tile width and kernel form never change results; the radix
  * plan changes them at the level of rounding. */
 int mfx_autotune(mfx_ctx *c, size_t n, int precision);
-/* set the column-pass variant of length L explicitly: the tile width (the
+/* set the column-pass variant of length L explicitly, for all uses of a direction
+ * (the projections go with the inverse one): the tile width (the
  * widest tile whose exchange area fits 64 KiB of LDS, half of it, or -- where
  * one workgroup can hold it -- twice it), or'ed with MFX_COL_PIPELINED for the
  * persistent pipelined kernel and with MFX_COL_PLAN_ALT for the length's

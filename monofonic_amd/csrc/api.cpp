@@ -1339,14 +1339,12 @@ int mfx_autotune(mfx_ctx* c, size_t n, int precision) {
     // the plain transform length n and the padded length 3n/2 of the
     // Orszag/LPT passes, where supported
     const int lens[2] = {(int)n, (int)(3 * n / 2)};
-    int tuned = 0;
-    for (int L : lens) {
-      if (!column_length_supported(L)) continue;
+    for (int q = 0; q < 2; ++q) {
+      if (!column_length_supported(lens[q])) continue;
       if (precision == MFX_FLOAT)
-        autotune_columns<float>(c->c, L);
+        autotune_columns<float>(c->c, lens[q], q == 1);
       else
-        autotune_columns<double>(c->c, L);
-      ++tuned;
+        autotune_columns<double>(c->c, lens[q], q == 1);
     }
     // lengths without tuned kernels run the generic kernels: nothing to tune
   });
@@ -1366,7 +1364,11 @@ int mfx_set_column_tile(mfx_ctx* c, int L, int precision, int inverse, int tile)
                     (cw > 0 ? " or " + std::to_string(cw) : std::string()) +
                     ", optionally or'ed with MFX_COL_PIPELINED" +
                     (column_plan_alt(L) ? " and MFX_COL_PLAN_ALT" : " (this length has one radix plan)"));
-    for (int cls = 0; cls < 2; ++cls) c->c.coltile[std::make_tuple(L, precision, inverse ? 1 : 0, cls)] = tile;
+    // every kind of pass in that direction; the turn passes end with the inverse one
+    const std::vector<int> kinds = inverse ? std::vector<int>{1, COL_PAD + 1, COL_HESS_Y, COL_TURN}
+                                           : std::vector<int>{0, COL_PAD, COL_TRUNC_OP};
+    for (int kind : kinds)
+      for (int cls = 0; cls < 2; ++cls) c->c.coltile[std::make_tuple(L, precision, kind, cls)] = tile;
   });
 }
 
@@ -1381,14 +1383,16 @@ int mfx_autotune_report(mfx_ctx* c, char* buf, size_t len) {
     for (const auto& r : c->c.tune_log) {
       std::snprintf(line, sizeof line, "L=%d %s %s%s:", r.L, r.tsize == 4 ? "f32" : "f64",
                     r.inv == COL_TURN ? "turn" : r.inv == COL_TRUNC_OP ? "truncating forward"
-                                                : (r.inv ? "inverse" : "forward"),
+                                                : (r.inv & 1 ? "inverse" : "forward"),
                     r.cls ? " plane-strided" : "");
       out += line;
       for (int q = 0; q < r.ncand; ++q) {
         std::snprintf(line, sizeof line, " %s %.4f ms%s", name(r.cand[q]).c_str(), r.ms[q], q + 1 < r.ncand ? "," : "");
         out += line;
       }
-      out += " -> " + name(r.chosen) + "\n";
+      out += " -> " + name(r.chosen);
+      if (r.hess) out += " (Hessian rows " + name(r.hess) + ")";
+      out += "\n";
     }
     std::snprintf(buf, len, "%s", out.c_str());
   });
@@ -1759,7 +1763,7 @@ extern "C" int mfx_icgen_create(mfx_ctx* c, const mfx_icgen_params* p, mfx_icgen
       if (p->autotune) {
         bool done = false;
         for (const auto& r : c->c.tune_log)
-          if (r.L == (int)(3 * p->n / 2) && r.tsize == p->precision) done = true;
+          if (r.L == (int)(3 * p->n / 2) && r.tsize == p->precision && r.inv == COL_TURN) done = true;
         if (!done) {
           int st = mfx_autotune(c, p->n, p->precision);
           if (st) throw Error(st, g_err);

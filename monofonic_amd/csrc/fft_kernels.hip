@@ -23,6 +23,8 @@
 #include "fft_passes.hpp"
 #include "ops.hpp"
 
+#include <algorithm>
+
 namespace mfx {
 
 // ------------------------------------------------------------------ 3D transforms
@@ -211,22 +213,29 @@ void conv2(Ctx& c, const cx<T>* fa, const MultSpec& ma, const cx<T>* fb, const M
 // budget keeps 8-16 adjacent columns per line access (wider HBM segments),
 // half of it doubles the workgroups per CU, twice it (where a workgroup can
 // hold it, in up to 160 KiB of LDS) doubles the run length again; the
-// persistent pipelined kernel
-// keeps the next tile's loads in flight while a tile is transformed; a
-// length's second radix plan (where it has one) trades an LDS exchange for
-// more elements per thread.  Which is faster depends on the length and
-// precision, so the (up to) twelve combinations are timed on a block of the library's own shape -- L/2+1
-// adjacent columns, up to 256 batches -- in both directions, five launches
-// each after two warm-ups, and the fastest is kept.  Lengths 3n/2 are timed on
-// the work grids' n/2 + 1 columns at their padded pitch, the only one that all
-// columns of a tile can be streamed to.
+// persistent pipelined kernel keeps the next tile's loads in flight while a tile
+// is transformed; a length's second radix plan (where it has one) trades an LDS
+// exchange for more elements per thread.  Which is faster depends on the length and
+// precision, so the (up to) twelve combinations are timed on passes of the library's
+// own shapes, five launches each after two warm-ups, and the fastest is kept.
+//   plain lengths: the in-place passes of a grid with rows of L/2+1 values, up to 256 of
+//     its planes: y passes row by row, x passes over a plane's columns as one range
+//   padded lengths 3n/2: the passes of the convolver and of the LPT engine on the work
+//     grids' n/2+1 columns and pitch
+// A length may be both; its two uses are timed and chosen apart.
 template <typename T>
-void autotune_columns(Ctx& c, int L) {
+void autotune_columns(Ctx& c, int L, bool padded) {
   const int cm = col_tile_max<T>(L);
-  const int ncols = L % 3 == 0 ? L / 3 + 1 : L / 2 + 1;
-  const int pitch = L % 3 == 0 ? conv_pitch(2 * L / 3) : ncols;
+  const int nn = 2 * L / 3;  // padded lengths: the grid's size
+  const int ncols = padded ? nn / 2 + 1 : L / 2 + 1;
+  const int pitch = padded ? conv_pitch(nn) : ncols;
   const int nb = L < 256 ? L : 256;
-  const long long cnt = (long long)nb * L * pitch;
+  // padded passes read and write arrays of their own, `sets` line sets of nn and of L
+  // values: as many as the grid has where it is small
+  const long long set = (long long)nn * pitch + (long long)L * pitch;
+  long long cnt = (long long)nb * L * pitch;
+  if (padded && nn <= 256) cnt = std::max(cnt, nn * set);
+  const int sets = padded ? (int)std::min<long long>(nn, cnt / set) : 0;
   cx<T>* buf = reinterpret_cast<cx<T>*>(c.alloc(sizeof(cx<T>) * cnt));
   hipEvent_t e0 = nullptr, e1 = nullptr;
   const bool prof = c.profile;
@@ -237,6 +246,7 @@ void autotune_columns(Ctx& c, int L) {
     MFX_HIP(hipEventCreate(&e1));
     // times every candidate variant of (direction, stride class) with
     // pass(), keeps the fastest and logs the timings
+    int hess = 0;
     auto tune = [&](int dir, int cls, bool alts, auto&& pass) {
       TuneRec rec{L, (int)sizeof(T), dir, cls, 0, {}, {}, cm};
       for (int alt = 0; alt < (alts && col_plan_alt(L) ? 2 : 1); ++alt) {
@@ -263,6 +273,11 @@ void autotune_columns(Ctx& c, int L) {
         }
       }
       c.coltile[std::make_tuple(L, (int)sizeof(T), dir, cls)] = rec.chosen;
+      if (dir == COL_HESS_Y) {
+        hess = rec.chosen;
+        return;
+      }
+      if (dir == COL_PAD + 1 && cls == 0) rec.hess = hess;
       c.tune_log.push_back(rec);
     };
     for (int cls = 0; cls < 2; ++cls) {
@@ -271,43 +286,48 @@ void autotune_columns(Ctx& c, int L) {
       // large enough to be class 1 at all
       const long long sb = cls ? pitch : (long long)L * pitch, sp = cls ? (long long)nb * pitch : pitch;
       if (stride_class(sp, (int)sizeof(cx<T>)) != cls) continue;
-      const bool padded = L % 3 == 0 && (L / 3) % 2 == 0;
-      const int nn = 2 * L / 3;
-      for (int inv = 0; inv < 2; ++inv) {
-        // at a padded length the row-strided inverse pass is the y stage of the
-        // Hessian rows: six outputs of three sources, as many planes as the block
-        // holds.  An in-place pass prefers other variants: 384-line FP64 1.94 ms of
-        // its choice against 1.00 to 1.35, 768-line FP32 4.72 against 4.15 (two fields)
-        const int planes = (int)((long long)nb * L / (3ll * nn + 6ll * L));
-        if (padded && inv && cls == 0 && planes > 0) {
+      if (!padded) {
+        const long long xb = cls ? 0 : sb;
+        const int xc = cls ? nb * ncols : ncols, xn = cls ? 1 : nb;
+        const SrcPlain<T> s{buf, xb, sp};
+        const DstPlain<T> d{buf, xb, sp, T(1)};
+        tune(0, cls, true, [&] { launch_col<T, false>(c, L, s, d, xc, xn, "tune", 0); });
+        tune(1, cls, true, [&] { launch_col<T, true>(c, L, s, d, xc, xn, "tune", 0); });
+        continue;
+      }
+      // the passes between the n lines at buf and the L lines behind them: the
+      // truncating forward pass and the inverse pass of padded lines
+      cx<T>* const m = buf + (long long)sets * nn * pitch;
+      const long long ns = cls ? pitch : (long long)nn * pitch, ms = cls ? pitch : (long long)L * pitch;
+      const long long ls = cls ? (long long)sets * pitch : pitch;
+      if (stride_class(ls, (int)sizeof(cx<T>)) == cls) {
+        const SrcPlain<T> fs{m, ms, ls};
+        const DstTrunc<T> fd{buf, ns, ls, nn};
+        tune(COL_PAD, cls, true, [&] { launch_col<T, false>(c, L, fs, fd, ncols, sets, "tune", 0); });
+        if (cls == 0) {
+          // six outputs of three sources, as many planes as the block holds
+          const int planes = (int)std::max<long long>(1, cnt / (pitch * (3ll * nn + 6ll * L)));
           const long long xs = (long long)planes * nn * pitch, ys = (long long)planes * L * pitch;
           cx<T>* const y = buf + 3 * xs;
           const SrcHessY<T> hs{{buf, buf + xs, buf + 2 * xs}, (long long)nn * pitch, pitch, nn, T(1)};
           const DstHessY<T> hd{{y, y + ys, y + 2 * ys, y + 3 * ys, y + 4 * ys, y + 5 * ys}, sb, sp};
-          tune(inv, cls, true, [&] { launch_hess_y<T>(c, L, hs, hd, ncols, planes, "tune", 0); });
-          continue;
+          tune(COL_HESS_Y, cls, true, [&] { launch_hess_y<T>(c, L, hs, hd, ncols, planes, "tune", 0); });
         }
-        tune(inv, cls, true, [&] {
-          if (inv)
-            launch_col<T, true>(c, L, SrcPlain<T>{buf, sb, sp}, DstPlain<T>{buf, sb, sp, T(1)}, ncols, nb, "tune", 0);
-          else
-            launch_col<T, false>(c, L, SrcPlain<T>{buf, sb, sp}, DstPlain<T>{buf, sb, sp, T(1)}, ncols, nb, "tune", 0);
-        });
+        const SrcPad<T, false> is{buf, ns, ls, nn, T(1), T(1), MultDev<T>{}};
+        const DstPlain<T> id{m, ms, ls, T(1)};
+        tune(COL_PAD + 1, cls, true, [&] { launch_col<T, true>(c, L, is, id, ncols, sets, "tune", 0); });
       }
-      // the projection (turn) passes of the padded lengths M = 3n/2, in place
-      // as in the LPT engine: two transforms per line and more registers than
-      // a plain pass, so they are tuned on their own
-      if (padded) {
-        const TurnArgs<T> ta{buf, sb, sp, nn, T(1), T(1), buf, sb, sp, nb, 0, 0};
-        tune(COL_TURN, cls, true, [&] { launch_turn<T>(c, L, ta, ncols, nb, "tune", 0); });
-        // the truncating forward pass with an output operator (the last x
-        // pass of a convolution or LPT source), in place: each workgroup
-        // writes only the retained positions of the lines it has read; these
-        // passes always run plan 0
-        DstTruncOp<T> dt{{buf}, nb, sb, sp, nn, OP_ASSIGN, T(0), T(1), 1, T(1)};
-        tune(COL_TRUNC_OP, cls, false,
-             [&] { launch_col<T, false>(c, L, SrcPlain<T>{buf, sb, sp}, dt, ncols, nb, "tune", 0); });
-      }
+      // the projection (turn) passes, in place as in the LPT engine: two transforms
+      // per line and more registers than a plain pass
+      const TurnArgs<T> ta{buf, sb, sp, nn, T(1), T(1), buf, sb, sp, nb, 0, 0};
+      tune(COL_TURN, cls, true, [&] { launch_turn<T>(c, L, ta, ncols, nb, "tune", 0); });
+      // the truncating forward pass with an output operator (the last x
+      // pass of a convolution or LPT source), in place: each workgroup
+      // writes only the retained positions of the lines it has read; these
+      // passes always run plan 0
+      DstTruncOp<T> dt{{buf}, nb, sb, sp, nn, OP_ASSIGN, T(0), T(1), 1, T(1)};
+      tune(COL_TRUNC_OP, cls, false,
+           [&] { launch_col<T, false>(c, L, SrcPlain<T>{buf, sb, sp}, dt, ncols, nb, "tune", 0); });
     }
   } catch (...) {
     c.profile = prof;
@@ -323,8 +343,8 @@ void autotune_columns(Ctx& c, int L) {
   c.release(buf);
 }
 
-template void autotune_columns<float>(Ctx&, int);
-template void autotune_columns<double>(Ctx&, int);
+template void autotune_columns<float>(Ctx&, int, bool);
+template void autotune_columns<double>(Ctx&, int, bool);
 
 int column_plan_alt(int L) { return col_plan_alt(L) ? 1 : 0; }
 

@@ -867,11 +867,43 @@ struct HeavyDst<DstTruncOp<T>> {
   static constexpr bool value = true;
 };
 
+// Passes over padded lines: out of place, on the work grids' pitch, where tiles stream
+// their stores.  The in-place passes of a plain grid of the same length have other
+// best variants (inverse y pass of 192 lines, FP32: 14.0 us with its own choice, 16.9
+// with that of the Hessian rows; x passes of 384, FP64: 153 and 157 us, 160 and 180 with
+// the choice for a row of columns at a time).
+template <class S>
+struct PaddedPass {
+  static constexpr bool value = false;
+};
+template <typename T, bool MULT>
+struct PaddedPass<SrcPad<T, MULT>> {
+  static constexpr bool value = true;
+};
+template <typename T>
+struct PaddedPass<DstTrunc<T>> {
+  static constexpr bool value = true;
+};
+template <class S>
+struct HessPass {
+  static constexpr bool value = false;
+};
+template <typename T>
+struct HessPass<SrcHessY<T>> {
+  static constexpr bool value = true;
+};
+
+// the kind a pass is tuned as
+template <bool INV, class Src, class Dst>
+constexpr int col_kind() {
+  if (HeavyDst<Dst>::value) return COL_TRUNC_OP;
+  if (HessPass<Src>::value) return COL_HESS_Y;
+  return (PaddedPass<Src>::value || PaddedPass<Dst>::value ? COL_PAD : 0) + (INV ? 1 : 0);
+}
+
 template <typename T, int L, bool INV, class Src, class Dst>
 void launch_col_L(Ctx& c, Src s, Dst d, int ncols, int nbatch, const char* name, double bytes) {
-  // register-heavy destinations have tuning decisions of their own
-  const int dir = HeavyDst<Dst>::value ? COL_TRUNC_OP : (INV ? 1 : 0);
-  const int v = c.col_tile(L, (int)sizeof(T), dir, ColCfg<T, L>::C, stride_class(s.sp, (int)sizeof(cx<T>)));
+  const int v = c.col_tile(L, (int)sizeof(T), col_kind<INV, Src, Dst>(), ColCfg<T, L>::C, stride_class(s.sp, (int)sizeof(cx<T>)));
   if constexpr (PlanAlt<L>::value && !HeavyDst<Dst>::value) {
     if (v & COL_PLAN_ALT) {
       launch_col_LV<T, L, INV, 1>(c, v, s, d, ncols, nbatch, name, bytes);
@@ -1113,7 +1145,7 @@ void launch_multi_LV(Ctx& c, int v, const M& a, int ncols, int nbatch, const cha
 // instead of 95 VGPRs, two waves per SIMD instead of five; plan 0 now takes 80)
 template <typename T, int L, bool INV, class M>
 void launch_multi_L(Ctx& c, const M& a, long long sp, int ncols, int nbatch, const char* name, double bytes) {
-  const int v = c.col_tile(L, (int)sizeof(T), INV, ColCfg<T, L>::C, stride_class(sp, (int)sizeof(cx<T>)));
+  const int v = c.col_tile(L, (int)sizeof(T), COL_PAD + (INV ? 1 : 0), ColCfg<T, L>::C, stride_class(sp, (int)sizeof(cx<T>)));
   launch_multi_LV<T, L, INV, 0>(c, v, a, ncols, nbatch, name, bytes);
 }
 

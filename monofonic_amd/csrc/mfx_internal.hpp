@@ -40,8 +40,12 @@ struct Error : std::runtime_error {
 constexpr int COL_PIPELINED = 0x100;
 constexpr int COL_PLAN_ALT = 0x200;  // the length's second radix plan
 constexpr int COL_WIDTH = 0xff;       // tile width bits of a column variant
-constexpr int COL_TURN = 2;           // tuning direction key of the turn (projection) passes
-constexpr int COL_TRUNC_OP = 3;       // tuning direction key of the truncating x passes with an output operator
+// Kinds of column pass that are tuned on their own: 0 and 1 the plain forward and
+// inverse pass, and of the padded lengths
+constexpr int COL_TURN = 2;      // the turn (projection) passes
+constexpr int COL_TRUNC_OP = 3;  // the truncating x passes with an output operator
+constexpr int COL_PAD = 4;       // the truncating forward passes; + 1 the inverse passes of padded lines
+constexpr int COL_HESS_Y = 6;    // the y stage of the Hessian rows
 // Stride class of a column pass: 0 when consecutive line elements are close
 // (the y passes, a row of kz columns apart), 1 when they are 64 KiB or more
 // apart (the x passes, a whole plane apart).  The two access patterns load
@@ -54,6 +58,7 @@ struct TuneRec {
   int cand[12];
   double ms[12];
   int chosen;
+  int hess = 0;  // the Hessian y stage's variant, logged with the padded row-strided inverse pass
 };
 
 // one profiled kernel launch
@@ -209,7 +214,7 @@ int conv_pitch(int n);
 // Times the column-pass tile candidates of line length L (both directions)
 // and stores the faster in c.coltile.  Throws for unsupported lengths.
 template <typename T>
-void autotune_columns(Ctx& c, int L);
+void autotune_columns(Ctx& c, int L, bool padded);
 // 1 if column passes of line length L are built
 int column_length_supported(int L);
 // widest tile of length L for element size tsize (4: FP32, 8: FP64)

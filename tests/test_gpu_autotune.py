@@ -169,3 +169,24 @@ def test_autotune_records_decisions():
         ctx.set_column_tile(512, "float", 0, 32)
     ctx.set_column_tile(768, "float", 0, 16 | PIPE | ALT)
     ctx.close()
+
+
+def test_uses_of_a_length_are_tuned_apart():
+    """192 is a plain length of 192^3 grids and the padded length of 128^3 ones, 96
+    that of 64^3 ones: neither use stands in for the other"""
+    import monofonic_amd as M
+    ctx = M.Context(0)
+
+    def lines(L):
+        return [ln for ln in ctx.autotune_report().splitlines() if ln.startswith(f"L={L} f32")]
+
+    ctx.autotune(192, "float")
+    assert len(lines(192)) == 4 and not any("turn" in ln or "truncating" in ln for ln in lines(192))
+    rows = [ln for ln in lines(288) if "inverse" in ln and "plane-strided" not in ln]
+    assert len(rows) == 1 and "Hessian rows C=" in rows[0]
+    ctx.autotune(96, "float")  # 96 and 144
+    assert not any("turn" in ln for ln in lines(96))
+    ic = M.ICGenerator(ctx, 64, 128.0, 24.0, LPTorder=2, precision="float", generator="NGENIC", seed=1)
+    assert sum("turn" in ln for ln in lines(96)) >= 1  # a generator of 64^3 times its padded passes
+    del ic
+    ctx.close()
