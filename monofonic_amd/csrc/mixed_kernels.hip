@@ -189,6 +189,25 @@ template const MixCfg& mix_cfg<float>(Ctx&, int, int);
 template const MixCfg& mix_cfg<double>(Ctx&, int, int);
 
 // ------------------------------------------------------------------ columns
+// The passes that only the fused engine runs, at lengths with a schedule (its own
+// condition); the others take the direct-DFT kernel where there is none.
+template <class Src>
+struct EnginePass {
+  static constexpr bool value = false;
+};
+template <typename T>
+struct EnginePass<SrcHessY<T>> {
+  static constexpr bool value = true;
+};
+template <typename T>
+struct EnginePass<SrcSplit<T>> {
+  static constexpr bool value = true;
+};
+template <typename T>
+struct EnginePass<MultiSrc<T, MultiPow<T>>> {
+  static constexpr bool value = true;
+};
+
 template <typename T, bool INV, class Src, class Dst>
 void launch_col_any(Ctx& c, int L, Src s, Dst d, int ncols, int nbatch, const char* name, double bytes) {
   const MixCfg& m = mix_cfg<T>(c, L, MIX_COL);
@@ -202,15 +221,19 @@ void launch_col_any(Ctx& c, int L, Src s, Dst d, int ncols, int nbatch, const ch
     check_launch(name);
     return;
   }
-  const GenPlan plan = gen_plan(L);
-  const int C = gen_col_tile<T>(L);
-  const size_t lds = 2 * (size_t)L * C * sizeof(cx<T>);
-  auto k = k_col_gen<T, INV, Src, Dst>;
-  col_lds_prep(c, k, lds);
-  LaunchScope ls(c, name, bytes);
-  hipLaunchKernelGGL(k, dim3((ncols + C - 1) / C, nbatch), dim3(GEN_THREADS), lds, c.stream, s, d, c.twiddles<T>(L),
-                     ncols, plan, C);
-  check_launch(name);
+  if constexpr (EnginePass<Src>::value) {
+    throw Error(1, "unsupported transform length " + std::to_string(L));
+  } else {
+    const GenPlan plan = gen_plan(L);
+    const int C = gen_col_tile<T>(L);
+    const size_t lds = 2 * (size_t)L * C * sizeof(cx<T>);
+    auto k = k_col_gen<T, INV, Src, Dst>;
+    col_lds_prep(c, k, lds);
+    LaunchScope ls(c, name, bytes);
+    hipLaunchKernelGGL(k, dim3((ncols + C - 1) / C, nbatch), dim3(GEN_THREADS), lds, c.stream, s, d, c.twiddles<T>(L),
+                       ncols, plan, C);
+    check_launch(name);
+  }
 }
 
 // only reached for lengths with a schedule: the fused engine runs no others
@@ -304,6 +327,7 @@ template <typename T>
 void launch_row_c2r_any(Ctx& c, int K, const cx<T>* src, long long spitch, int hin, T* dst, long long dpitch,
                         long long nrows, T scale, const char* name, double bytes) {
   const MixCfg& m = mix_cfg<T>(c, 2 * K, MIX_ROW);
+  MFX_REQUIRE(!m.ok || hin == K + 1, "the row kernel reads whole half spectra");
   if (m.ok)
     MFX_MIX_ROW(k_mix_c2r, m, src, spitch, hin, dst, dpitch, scale);
   else
@@ -314,6 +338,7 @@ template <typename T>
 void launch_row_c2r_part_any(Ctx& c, int K, const cx<T>* src, long long spitch, int hin, const PartOut& po,
                              long long nrows, T scale, double lunit, double qoff, const char* name, double bytes) {
   const MixCfg& m = mix_cfg<T>(c, 2 * K, MIX_ROW);
+  MFX_REQUIRE(!m.ok || hin == K + 1, "the row kernel reads whole half spectra");
   if (m.ok)
     MFX_MIX_ROW(k_mix_c2r_part, m, src, spitch, hin, po, scale, lunit, qoff);
   else

@@ -649,9 +649,9 @@ struct Ranlxd {
   int ir, jr, ir_old, pr;
 };
 
-__host__ __device__ __forceinline__ int rl_next(int i) { return i == 11 ? 0 : i + 1; }
+__device__ __forceinline__ int rl_next(int i) { return i == 11 ? 0 : i + 1; }
 
-__host__ __device__ void rl_seed(Ranlxd& s, unsigned long seed) {
+__device__ void rl_seed(Ranlxd& s, unsigned long seed) {
   const double one_bit = 1.0 / 281474976710656.0;
   int xbit[31];
   if (seed == 0) seed = 1;
@@ -681,7 +681,7 @@ __host__ __device__ void rl_seed(Ranlxd& s, unsigned long seed) {
 }
 
 // one carry step on x[ir] -= x[jr] convention of RANLUX
-__host__ __device__ void rl_increment(Ranlxd& s) {
+__device__ void rl_increment(Ranlxd& s) {
   const double one_bit = 1.0 / 281474976710656.0;
   double carry = s.carry;
   int ir = s.ir, jr = s.jr;
@@ -706,7 +706,7 @@ __host__ __device__ void rl_increment(Ranlxd& s) {
   s.carry = carry;
 }
 
-__host__ __device__ __forceinline__ double rl_uniform(Ranlxd& s) {
+__device__ __forceinline__ double rl_uniform(Ranlxd& s) {
   int ir = s.ir;
   s.ir = rl_next(ir);
   if (s.ir == s.ir_old) rl_increment(s);
