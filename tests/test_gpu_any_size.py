@@ -1,7 +1,7 @@
 """Grid sizes without tuned kernels (the reference plans any size through
-FFTW, src/grid_fft.cc:43-112): the generic runtime-plan transforms
-(fft_generic.hpp) against numpy's rfftn, and whole IC realisations at such
-sizes against the oracle."""
+FFTW, src/grid_fft.cc:43-112): the run-time schedules (fft_mixed.hpp, and
+fft_generic.hpp for prime factors above 7) against numpy's rfftn, and whole IC
+realisations at such sizes against the oracle."""
 import numpy as np
 import pytest
 
@@ -38,7 +38,8 @@ def test_r2c_any_length_vs_numpy(ctx, shape, prec, tol):
                                                   (80, 2, "float", 1e-5), (320, 2, "float", 1e-5)])
 def test_icgen_any_size_vs_oracle(ctx, orc, n, order, prec, rms_tol):
     """NGENIC realisations at grid sizes 160, 200 (padded 240, 300), 80 and
-    320 (padded 120, 480): the convolve sequence on the generic transforms"""
+    320 (padded 120, 480): the mixed-radix transforms and, above first order, the
+    fused engine on its mixed-radix z stages"""
     import monofonic_amd as M
     from test_gpu_configs import compare_fields
     from test_gpu_lpt import oracle_pipeline

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n,prec", [(16, "float"), (64, "double"), (160, "float"), (160, "double"), (192, "float"),
-                                    (192, "double"), (44, "float")])
+                                    (192, "double"), (224, "double"), (44, "float")])
 def test_particle_components_equal_one_at_a_time(ctx, n, prec):
     """with baryons every component is transformed on its own, from the same
     assembled values and by the same kernels: the same bits"""
