@@ -352,7 +352,7 @@ __device__ __forceinline__ void fft_exec(cx<T> (&v)[EPT], cx<T>* lds, int ls, in
   stage_loop<T, L, INV, 0, V>(v, lds, ls, t, global_table(tw), w0);
 }
 
-// fft_exec with the twiddle table copied to LDS at twl (TwCount entries,
+// fft_exec with the twiddle table copied to LDS at twl (tw_count entries,
 // visible to every thread: the copy is followed by a barrier before the first
 // call)
 template <typename T, int L, bool INV, int V = 0, int EPT>

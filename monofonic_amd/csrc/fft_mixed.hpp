@@ -499,7 +499,9 @@ __global__ void __launch_bounds__(1024)
 // Two real rows A and B are one complex line A + i B of the full length M: its
 // transform needs no half-length split step, no second twiddle table and no
 // even M / 2, and a workgroup holds `pairs` such lines.  The half spectra
-// combine as Z[k] = A[k] + i B[k], Z[M - k] = conj(A[k]) + i conj(B[k]).
+// combine as Z[k] = A[k] + i B[k], Z[M - k] = conj(A[k]) + i conj(B[k]).  The price is
+// precision of the smaller row: both are rounded at the size of the larger one (rows
+// of a pair are neighbours of a field), and taking them apart rounds once more.
 struct MixRowArgs {
   MixPlan p;
   MixDiv nthr;  // threads per pair
