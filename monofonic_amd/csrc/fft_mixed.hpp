@@ -42,9 +42,10 @@ namespace mfx {
 // where such sums are subtracted again the rounding stays in the output.  Radices 2,
 // 4, 8 and 12 form the outputs k = +-1 from differences of values, and so do 6 and 10
 // with their radix 2 first; an odd radix does it only from differences with one of
-// its values (mix_first_bf).  A line of mean 1 with 1 % fluctuations, 240 points in
-// single precision, rms error of k = 1 in units of 2^-24 of the fluctuations: 1.3 with 8
-// first, 1.5 with this 10, 43 with a 10 whose 5-point parts take raw values.
+// its values (mix_first_bf: the first butterfly of a forward transform).  A line of
+// mean 1 with 1 % fluctuations, 240 points in single precision, rms error of k = 1 in
+// units of 2^-24 of the fluctuations: 1.3 with 8 first, 1.5 with 10 first in that form,
+// 43 with a 10 whose 5-point parts take raw values.
 template <int R, bool INV, typename T>
 struct MixBF : BF<R, INV, T> {};
 
@@ -126,30 +127,49 @@ struct MixBF<7, INV, T> {
   static __device__ __forceinline__ void run(cx<T>* a) { mix7<INV, T, false>(a); }
 };
 
-// 2 P for an odd P without inner twiddles, the radix 2 first: inputs
-// 2 n1 + P n2, output k = k1 mod P = k2 mod 2
-template <int P, bool INV, typename T>
-struct MixTwice {
-  static __device__ __forceinline__ void run(cx<T>* a) {
-    cx<T> t[2][P];
+// 2 P for an odd P without inner twiddles: inputs 2 n1 + P n2, output k = k1 mod P =
+// k2 mod 2.  TWO: the radix 2 first
+template <int P, bool INV, typename T, bool TWO>
+__device__ __forceinline__ void mix_twice(cx<T>* a) {
+  cx<T> t[2][P];
+#pragma unroll
+  for (int n1 = 0; n1 < P; ++n1) {
+    t[0][n1] = a[(2 * n1) % (2 * P)];
+    t[1][n1] = a[(2 * n1 + P) % (2 * P)];
+  }
+  auto two = [&] {
 #pragma unroll
     for (int n1 = 0; n1 < P; ++n1) {
-      const cx<T> u = a[(2 * n1) % (2 * P)], v = a[(2 * n1 + P) % (2 * P)];
+      const cx<T> u = t[0][n1], v = t[1][n1];
       t[0][n1] = u + v;
       t[1][n1] = u - v;
     }
-#pragma unroll
-    for (int k2 = 0; k2 < 2; ++k2) {
-      MixBF<P, INV, T>::run(t[k2]);
-#pragma unroll
-      for (int k1 = 0; k1 < P; ++k1) a[k1 % 2 == k2 ? k1 : k1 + P] = t[k2][k1];
-    }
+  };
+  auto odd = [&] {
+    MixBF<P, INV, T>::run(t[0]);
+    MixBF<P, INV, T>::run(t[1]);
+  };
+  if constexpr (TWO) {
+    two();
+    odd();
+  } else {
+    odd();
+    two();
   }
+#pragma unroll
+  for (int k2 = 0; k2 < 2; ++k2) {
+#pragma unroll
+    for (int k1 = 0; k1 < P; ++k1) a[k1 % 2 == k2 ? k1 : k1 + P] = t[k2][k1];
+  }
+}
+template <bool INV, typename T>
+struct MixBF<6, INV, T> {
+  static __device__ __forceinline__ void run(cx<T>* a) { mix_twice<3, INV, T, false>(a); }
 };
 template <bool INV, typename T>
-struct MixBF<6, INV, T> : MixTwice<3, INV, T> {};
-template <bool INV, typename T>
-struct MixBF<10, INV, T> : MixTwice<5, INV, T> {};
+struct MixBF<10, INV, T> {
+  static __device__ __forceinline__ void run(cx<T>* a) { mix_twice<5, INV, T, false>(a); }
+};
 
 // radix 9 as 3 x 3 with the inner twiddles W9^(n2 k1)
 template <bool INV, typename T, bool FIRST>
@@ -190,7 +210,7 @@ struct MixBF<9, INV, T> {
 // the butterfly of a line's raw values: the first of a forward transform
 template <int R, bool INV, typename T>
 __device__ __forceinline__ void mix_first_bf(cx<T>* a) {
-  if constexpr (INV || R % 2 == 0)
+  if constexpr (INV)
     MixBF<R, INV, T>::run(a);
   else if constexpr (R == 3)
     mix3<INV, T, true>(a);
@@ -198,8 +218,12 @@ __device__ __forceinline__ void mix_first_bf(cx<T>* a) {
     mix5<INV, T, true>(a);
   else if constexpr (R == 7)
     mix7<INV, T, true>(a);
-  else
+  else if constexpr (R == 9)
     mix9<INV, T, true>(a);
+  else if constexpr (R == 6 || R == 10)
+    mix_twice<R / 2, INV, T, true>(a);
+  else
+    MixBF<R, INV, T>::run(a);
 }
 
 // ---------------------------------------------------------------- schedule
@@ -736,7 +760,12 @@ struct MixZ {
     cx<T> v[S];
 #pragma unroll
     for (int q = 0; q < S; ++q) v[q] = w[q];
-    mix_first_bf<S, false, T>(v);
+    // FP32 products come without their mean (launch_row_mean); the engine's rows have
+    // none, or one of the size of their fluctuations
+    if constexpr (S % 2 == 1)
+      mix_first_bf<S, false, T>(v);
+    else
+      MixBF<S, false, T>::run(v);
     const int t = thread();
     if (t < r.nthr) {
 #pragma unroll

@@ -355,7 +355,7 @@ static bool mix_prod_rows(const MixCfg& m, int K, int hin) { return m.ok && hin 
 // the few per cent that MIX_MEAN_ROWS rows give) taken off before the transform and
 // added to the k = 0 mode after it, the rounding is that of the rest.  The 2LPT source
 // of a 160^3 FP32 grid by separate convolutions, median and maximum error over 20
-// seeds: 2.9e-7 and 3.5e-7, with the mean 7.8e-7 and 1.5e-6; of 240^3 3.5e-7 and 4.3e-7,
+// seeds: 3.1e-7 and 3.5e-7, with the mean 7.8e-7 and 1.5e-6; of 240^3 3.4e-7 and 4.3e-7,
 // with it 1.4e-6 and 2.0e-6.  The launch takes 5 us a product (160^3: 180 us).  FP64
 // results err by 1e-15 either way.
 template <typename T>
